@@ -321,8 +321,8 @@ bool wide_serves(const GemmParams &p, int bn, bool a_tr, bool b_tr) {
   if (p.M <= 0 || p.N <= 0 || p.K < 128 || p.N % 8 || p.rz || !packed_epilogue(p) || (a_tr && host_has_tail(p))) return false;
   if (p.K % 64 && !b_tr) return false;
   if (p.K % 8 && !a_tr) return false;
-  const bool a_fits = a_tr ? p.M % 8 == 0 && p.a_sk > 0 && ((int64_t)p.K + 64) * p.a_sk * 2 < limit : p.a_sm > 0 && p.a_sm * 2 * 256 < limit;
-  const bool b_fits = b_tr ? p.b_sk > 0 && ((int64_t)p.K + 64) * p.b_sk * 2 < limit : p.b_sn > 0 && p.b_sn * 2 * bn < limit;
+  const bool a_fits = a_tr ? p.M % 8 == 0 && p.a_sk > 0 && ((int64_t)p.K + 64) * p.a_sk * 2 < limit : p.a_sm > 0 && p.a_sm * 2 * 256 + (int64_t)p.K * 2 < limit;
+  const bool b_fits = b_tr ? p.b_sk > 0 && ((int64_t)p.K + 64) * p.b_sk * 2 < limit : p.b_sn > 0 && p.b_sn * 2 * bn + (int64_t)p.K * 2 < limit;
   return a_fits && b_fits && ((int64_t)(p.M + 255) / 256) * ((p.N + bn - 1) / bn) < limit;
 }
 

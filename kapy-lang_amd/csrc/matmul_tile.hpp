@@ -354,7 +354,7 @@ struct PackedEpilogue {
         const int voff = (int)(voff0 + (uint32_t)(i * 32 + t * kRowsPerPass) * pitch);
         if constexpr (OUT == 2) {
 #pragma unroll
-          for (int h = 0; h < kCols / 4; ++h) {  // (the scalar offset is outside the range check: the piece is in or out whole)
+          for (int h = 0; h < kCols / 4; ++h) {  // (in or out whole, whether or not the range check counts the scalar offset)
             u32x4 w;
 #pragma unroll
             for (int e = 0; e < 4; ++e) w[e] = __float_as_uint(v[4 * h + e]);

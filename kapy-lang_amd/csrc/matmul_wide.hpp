@@ -20,6 +20,7 @@
 // 0.84 ms for the turns and the product -> 0.74.
 #pragma once
 #include "matmul_tile.hpp"
+#include "operand_pieces.hpp"
 
 namespace kapy {
 namespace {
@@ -89,37 +90,36 @@ __global__ __launch_bounds__(256) void wide_kernel(GemmParams p) {
   // elements between neighbours along the staged rows' other extent: between rows (K-contiguous) or between k-rows (transposed)
   const int32_t a_ld = __builtin_amdgcn_readfirstlane((int32_t)(A_TR ? p.a_sk : p.a_sm)), b_ld = __builtin_amdgcn_readfirstlane((int32_t)(B_TR ? p.b_sk : p.b_sn));
 
-  // Per-lane global byte offset of the 16-byte piece this lane fetches with load instruction 0 of an operand; instruction q fills
-  // bytes [(wave + 4q) * 1024, + 1024) of the operand's image, which is 32 rows (K-contiguous) or 16 k-rows and, from q = 4 on, the
-  // other 128 rows or columns (transposed) further on - no key mixes in a bit that q changes - so the rest of an instruction's
-  // address is a scalar.
+  // Per-lane global byte offsets of the 16-byte pieces this lane fetches, one per load instruction: instruction q of an operand fills
+  // bytes [(wave + 4q) * 1024, + 1024) of its image, 32 rows (K-contiguous) or 16 k-rows and, from q = 4 on, the other 128 rows or
+  // columns (transposed) further on than instruction 0's - no key mixes in a bit that q changes.
   const uint32_t my_byte = (uint32_t)wave * 1024u + lane * 16u;
   uint32_t kc_row, kc_chunk;
   L::locate(my_byte, kc_row, kc_chunk);
   const uint32_t tr_krow = my_byte / kRowTr, tr_chunk = ((my_byte % kRowTr) / 16) ^ wide_key(tr_krow);
-  constexpr int kGoffA = KTAIL && A_TR ? 4 : 1, kGoffB = KTAIL && B_TR ? 4 : 1;
-  uint32_t a_goff[kGoffA], b_goff[kGoffB];
+  // (the lines and pieces a tile that hangs over an edge reads in place of those that do not exist: operand_pieces.hpp)
+  using PiecesA = OperandPieces<A_TR, BK, EB>;
+  using PiecesB = OperandPieces<B_TR, BK, EB>;
+  auto line_of = [&](bool tr, int q) -> uint32_t { return tr ? tr_krow + 16 * (q % 4) : kc_row + 32 * q; };
+  auto first_of = [&](bool tr, int q) -> uint32_t { return tr ? tr_chunk * 8 + 128 * (q / 4) : kc_chunk * (16 / EB); };
+  uint32_t a_goff[kLoadsA], b_goff[kLoadsB];
 #pragma unroll
-  for (int q = 0; q < kGoffA; ++q) a_goff[q] = A_TR ? (tr_krow * a_ld + tr_chunk * 8) * EB : kc_row * a_ld * EB + kc_chunk * 16;
+  for (int q = 0; q < kLoadsA; ++q) a_goff[q] = PiecesA::lane(line_of(A_TR, q), first_of(A_TR, q), a_ld, p.M - m0);
 #pragma unroll
-  for (int q = 0; q < kGoffB; ++q) b_goff[q] = B_TR ? (tr_krow * b_ld + tr_chunk * 8) * EB : kc_row * b_ld * EB + kc_chunk * 16;
+  for (int q = 0; q < kLoadsB; ++q) b_goff[q] = PiecesB::lane(line_of(B_TR, q), first_of(B_TR, q), b_ld, p.N - n0);
   auto enter_k_tail = [&]() __attribute__((always_inline)) {
     const int32_t k_left = p.K - (KT - 1) * BK;
 #pragma unroll
-    for (int q = 0; q < kGoffA; ++q) a_goff[q] = (A_TR ? (int32_t)tr_krow + 16 * q : (int32_t)kc_chunk * 8) >= k_left ? 0x7fffffffu : a_goff[q];
+    for (int q = 0; q < kLoadsA; ++q) a_goff[q] = PiecesA::beyond_k(line_of(A_TR, q), first_of(A_TR, q), k_left) ? PiecesA::kNowhere : a_goff[q];
 #pragma unroll
-    for (int q = 0; q < kGoffB; ++q) b_goff[q] = (B_TR ? (int32_t)tr_krow + 16 * q : (int32_t)kc_chunk * 8) >= k_left ? 0x7fffffffu : b_goff[q];
+    for (int q = 0; q < kLoadsB; ++q) b_goff[q] = PiecesB::beyond_k(line_of(B_TR, q), first_of(B_TR, q), k_left) ? PiecesB::kNowhere : b_goff[q];
   };
   auto uniform_ptr = [](const char *ptr) {
     const uint64_t v = (uint64_t)ptr;
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return (void *)(((uint64_t)hi << 32) | lo);
   };
-  // (the descriptors end where the operands end: of a tile that hangs over an edge, the rows of a K-contiguous operand that do not
-  // exist read as zeros; the rows or columns of a transposed one read the first elements of the next k-row, or zeros behind the
-  // last; either way they only reach results that are not stored)
-  const int64_t a_left = A_TR ? ((int64_t)(p.K - 1) * p.a_sk + (p.M - m0)) * EB : ((int64_t)(p.M - m0 - 1) * p.a_sm + p.K) * EB;
-  const int64_t b_left = B_TR ? ((int64_t)(p.K - 1) * p.b_sk + (p.N - n0)) * EB : ((int64_t)(p.N - n0 - 1) * p.b_sn + p.K) * EB;
+  const int64_t a_left = PiecesA::bytes(p.K, A_TR ? p.a_sk : p.a_sm, p.M - m0), b_left = PiecesB::bytes(p.K, B_TR ? p.b_sk : p.b_sn, p.N - n0);
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(p.a + (int64_t)m0 * (A_TR ? 1 : p.a_sm) * EB), 0,
                                                                           __builtin_amdgcn_readfirstlane((int)(a_left < 0x7fffffff ? a_left : 0x7fffffff)), 0x00020000);
   const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(p.b + (int64_t)n0 * (B_TR ? 1 : p.b_sn) * EB), 0,
@@ -127,18 +127,15 @@ __global__ __launch_bounds__(256) void wide_kernel(GemmParams p) {
   const int wave_lds = wave * 1024;
   // load instruction idx (the lhs ones, then the rhs ones) of this wavefront for the K-tile at scalar offsets soff_a / soff_b
   auto issue_load = [&](int soff_a, int soff_b, int stage, int idx) __attribute__((always_inline)) {
-    if (idx < kLoadsA) {
-      const int add = A_TR ? ((idx % 4) * 16 * a_ld + (idx / 4) * 128) * EB : idx * 32 * a_ld * EB;
+    if (idx < kLoadsA)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (__attribute__((address_space(3))) void *)(lds + stage * kStageBytes + idx * 4096 + wave_lds), 16,
-                                               (int)a_goff[idx % kGoffA], soff_a + add, 0, 0);
-    } else {
-      const int q = idx - kLoadsA, add = B_TR ? ((q % 4) * 16 * b_ld + (q / 4) * 128) * EB : q * 32 * b_ld * EB;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, (__attribute__((address_space(3))) void *)(lds + stage * kStageBytes + kImageB + q * 4096 + wave_lds), 16,
-                                               (int)b_goff[q % kGoffB], soff_b + add, 0, 0);
-    }
+                                               (int)a_goff[idx], soff_a, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, (__attribute__((address_space(3))) void *)(lds + stage * kStageBytes + kImageB + (idx - kLoadsA) * 4096 + wave_lds),
+                                               16, (int)b_goff[idx - kLoadsA], soff_b, 0, 0);
   };
-  auto soff_a_of = [&](int j) { return min(j, KT - 1) * BK * (A_TR ? a_ld : 1) * EB; };  // (tiles past the end of K repeat the last
-  auto soff_b_of = [&](int j) { return min(j, KT - 1) * BK * (B_TR ? b_ld : 1) * EB; };  //  one, into a stage nobody reads again)
+  auto soff_a_of = [&](int j) { return PiecesA::tile(j, KT, a_ld); };
+  auto soff_b_of = [&](int j) { return PiecesB::tile(j, KT, b_ld); };
 
   // Operand reads, from the operand fragments of the instruction.  K-contiguous: row frag.row of each KM-row block, the 16-byte chunks
   // that hold its kpack consecutive K elements of the slice.  Transposed: the transposing read hands lane j of a 16-lane group

@@ -546,10 +546,10 @@ int matmul_16bit(const kapy_global *lhs, const kapy_global *rhs, const kapy_glob
   }
   // An operand that is contiguous along its other extent - a row-major rhs (with a row-major lhs: the reference fixture's
   // layout, matmul.mlir), a column-major lhs - is staged as it lies and read with the transposing read.
-  const bool a_kc = p.a_sk == 1 && vector_bytes(lhs, 1) == 16 && p.a_sm >= 0 && p.a_sm * 2 * kNBM < (int64_t(1) << 31);
+  const bool a_kc = p.a_sk == 1 && vector_bytes(lhs, 1) == 16 && p.a_sm >= 0 && p.a_sm * 2 * kNBM + (int64_t)p.K * 2 < (int64_t(1) << 31);
   const bool a_tr = !a_kc && p.a_sm == 1 && vector_bytes(lhs, 0) == 16 && p.a_sk >= 0 && p.M % 8 == 0 && (int64_t)p.K * p.a_sk * 2 < (int64_t(1) << 31);
   const bool b_tr = p.b_sn == 1 && vector_bytes(rhs, 1) == 16 && p.b_sk >= 0 && (int64_t)p.K * p.b_sk * 2 < (int64_t(1) << 31);
-  const bool b_kc = !b_tr && p.b_sk == 1 && vector_bytes(rhs, 0) == 16 && p.b_sn >= 0 && p.b_sn * 2 * kNBN < (int64_t(1) << 31);
+  const bool b_kc = !b_tr && p.b_sk == 1 && vector_bytes(rhs, 0) == 16 && p.b_sn >= 0 && p.b_sn * 2 * kNBN + (int64_t)p.K * 2 < (int64_t(1) << 31);
   bool nn = (a_kc || a_tr) && (b_kc || b_tr) && (a_tr || b_tr || p.K % 8) && p.M > 0 && p.K > 0 &&
             c.impl_way != KAPY_MFMA_32X32X16_16B && (!c.tile_m || c.tile_m == kNBM) && (!c.tile_n || c.tile_n == kNBN) && (!c.waves || c.waves == 4);
   if (nn) {

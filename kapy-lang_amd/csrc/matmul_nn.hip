@@ -1,5 +1,6 @@
 // matmul_nn.hip — the tiled kernel for 16-bit operands of which at least one is contiguous along its other extent (128 x 128 tiles).
 #include "matmul_tile.hpp"
+#include "operand_pieces.hpp"
 
 namespace kapy {
 namespace {
@@ -53,40 +54,42 @@ __global__ __launch_bounds__(256) void nn_kernel(GemmParams p) {
   // elements between neighbours along the staged rows' other extent: between rows (K-contiguous) or between k-rows (transposed)
   const int32_t a_ld = (int32_t)(A_TR ? p.a_sk : p.a_sm), b_ld = (int32_t)(B_TR ? p.b_sk : p.b_sn);
 
-  // Per-lane global byte offsets of the 16-byte chunks this lane fetches, one per load instruction (instruction q of an operand
-  // fills LDS bytes [q*1024, q*1024 + 1024) of its image).
-  auto goff_of = [&](bool tr, int q, int32_t ld) -> uint32_t {
+  // Per-lane global byte offsets of the 16-byte pieces this lane fetches, one per load instruction (instruction q of an operand
+  // fills LDS bytes [q*1024, q*1024 + 1024) of its image), with what a tile that hangs over an edge reads in place of rows, columns
+  // and pieces that do not exist (operand_pieces.hpp).
+  using PiecesA = OperandPieces<A_TR, BK, 2>;
+  using PiecesB = OperandPieces<B_TR, BK, 2>;
+  // row or k-row, and first element along it, of the piece that instruction q of an operand brings this lane
+  auto piece_of = [&](bool tr, int q, uint32_t &line, uint32_t &first) {
     const uint32_t o = (uint32_t)(wave + q * 4) * 1024u + lane * 16u;
-    uint32_t row, chunk;
+    uint32_t chunk;
     if (tr) {
-      row = o / kRowTr;
-      chunk = ((o % kRowTr) / 16) ^ rhs_key(row);
+      line = o / kRowTr;
+      chunk = ((o % kRowTr) / 16) ^ rhs_key(line);
     } else {
-      LA::locate(o, row, chunk);
+      LA::locate(o, line, chunk);
     }
-    return (uint32_t)((row * ld + chunk * 8) * 2);
+    first = chunk * 8;
   };
   uint32_t a_goff[kLoadsOp], b_goff[kLoadsOp];
 #pragma unroll
   for (int q = 0; q < kLoadsOp; ++q) {
-    a_goff[q] = goff_of(A_TR, q, a_ld);
-    b_goff[q] = goff_of(B_TR, q, b_ld);
+    uint32_t line, first;
+    piece_of(A_TR, q, line, first);
+    a_goff[q] = PiecesA::lane(line, first, a_ld, p.M - m0);
+    piece_of(B_TR, q, line, first);
+    b_goff[q] = PiecesB::lane(line, first, b_ld, p.N - n0);
   }
-  // (KTAIL) first K position, within a tile, of the piece that load instruction q of an operand brings this lane
-  auto k_of = [&](bool tr, int q) -> int32_t {
-    const uint32_t o = (uint32_t)(wave + q * 4) * 1024u + lane * 16u;
-    uint32_t row, chunk;
-    if (tr) return (int32_t)(o / kRowTr);
-    LA::locate(o, row, chunk);
-    return (int32_t)chunk * 8;
-  };
   // From the last K-tile on (the loads past the end of K repeat it): pieces at or beyond K get an offset no descriptor covers.
   auto enter_k_tail = [&]() __attribute__((always_inline)) {
     const int32_t k_left = p.K - (KT - 1) * BK;
 #pragma unroll
     for (int q = 0; q < kLoadsOp; ++q) {
-      a_goff[q] = k_of(A_TR, q) >= k_left ? 0x7fffffffu : a_goff[q];
-      b_goff[q] = k_of(B_TR, q) >= k_left ? 0x7fffffffu : b_goff[q];
+      uint32_t line, first;
+      piece_of(A_TR, q, line, first);
+      a_goff[q] = PiecesA::beyond_k(line, first, k_left) ? PiecesA::kNowhere : a_goff[q];
+      piece_of(B_TR, q, line, first);
+      b_goff[q] = PiecesB::beyond_k(line, first, k_left) ? PiecesB::kNowhere : b_goff[q];
     }
   };
   // (KTAIL) Of a K-contiguous operand the piece that K ends inside has arrived with what lies behind K: this lane's copy of it in the
@@ -97,9 +100,11 @@ __global__ __launch_bounds__(256) void nn_kernel(GemmParams p) {
 #pragma unroll
     for (int q = 0; q < kLoadsOp; ++q) {
       char *piece = lds + stage * kStage + q * 4096 + wave * 1024 + lane * 16;
+      uint32_t line, first;
+      piece_of(false, q, line, first);
 #pragma unroll
       for (int e = 1; e < 8; ++e) {
-        const int32_t from = k_left - k_of(false, q);   // (one compare per element: the piece K ends inside has 1 .. 7 left)
+        const int32_t from = k_left - (int32_t)first;   // (one compare per element: the piece K ends inside has 1 .. 7 left)
         if (from > 0 && from <= e) {
           if constexpr (!A_TR) ((uint16_t *)piece)[e] = 0;
           if constexpr (!B_TR) ((uint16_t *)(piece + kBytesA))[e] = 0;
@@ -112,26 +117,15 @@ __global__ __launch_bounds__(256) void nn_kernel(GemmParams p) {
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return (void *)(((uint64_t)hi << 32) | lo);
   };
-  // The lhs descriptor ends where the lhs ends: a tile of a K-contiguous lhs that hangs over its last rows (M not a multiple of
-  // 128) gets zeros for the rows that do not exist (their per-lane offsets are out of range) instead of a fault.  (Of a
-  // transposed lhs - M a multiple of 8 - the rows that do not exist are the first elements of the next k-row, or zeros behind
-  // the last one; they only reach results that are not stored.)
-  // (A line whose length is no multiple of 8 ends inside an aligned 16-byte piece, which is loaded whole: the descriptors end with
-  // that piece.)
-  auto whole_pieces = [](int64_t bytes) { return (bytes + 15) & ~int64_t(15); };
-  const int64_t a_left = whole_pieces(A_TR ? ((int64_t)(p.K - 1) * p.a_sk + (p.M - m0)) * 2 : ((int64_t)(p.M - m0 - 1) * p.a_sm + p.K) * 2);
+  const int64_t a_left = PiecesA::bytes(p.K, A_TR ? p.a_sk : p.a_sm, p.M - m0), b_left = PiecesB::bytes(p.K, B_TR ? p.b_sk : p.b_sn, p.N - n0);
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(p.a + (int64_t)m0 * (A_TR ? 1 : p.a_sm) * 2), 0,
                                                                           __builtin_amdgcn_readfirstlane((int)(a_left < 0x7fffffff ? a_left : 0x7fffffff)), 0x00020000);
-  // The rhs descriptor ends where the rhs ends, too: of a tile that hangs over the last columns (N not a multiple of 128) the
-  // columns that do not exist read zeros or, in a transposed rhs, the first elements of the next k-row; either way they only
-  // reach results that are not stored.
-  const int64_t b_left = whole_pieces(B_TR ? ((int64_t)(p.K - 1) * p.b_sk + (p.N - n0)) * 2 : ((int64_t)(p.N - n0 - 1) * p.b_sn + p.K) * 2);
   const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(p.b + (int64_t)n0 * (B_TR ? 1 : p.b_sn) * 2), 0,
                                                                           __builtin_amdgcn_readfirstlane((int)(b_left < 0x7fffffff ? b_left : 0x7fffffff)), 0x00020000);
   const int wave_lds = wave * 1024;
   // (the scalar offsets of K-tile j, clamped to the last tile: loads past the end of K are still issued, into stages nobody reads)
-  auto soff_a_of = [&](int j) { return min(j, KT - 1) * BK * (A_TR ? a_ld : 1) * 2; };
-  auto soff_b_of = [&](int j) { return min(j, KT - 1) * BK * (B_TR ? b_ld : 1) * 2; };
+  auto soff_a_of = [&](int j) { return PiecesA::tile(j, KT, a_ld); };
+  auto soff_b_of = [&](int j) { return PiecesB::tile(j, KT, b_ld); };
   auto issue_load_at = [&](int soff_a, int soff_b, int stage, int idx) __attribute__((always_inline)) {
     if (idx < kLoadsOp)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (__attribute__((address_space(3))) void *)(lds + stage * kStage + idx * 4096 + wave_lds), 16,
@@ -317,8 +311,8 @@ __global__ __launch_bounds__(256) void nn_kernel(GemmParams p) {
 
 template <typename T, int BK, int STAGES, bool A_TR = false, bool B_TR = true, bool KTAIL = false>
 int launch_nn(GemmParams p, hipStream_t s) {
-  p.tiles_m = (p.M + kNBM - 1) / kNBM;  // (a K-contiguous lhs need not have whole tiles of rows: see the kernel's lhs descriptor)
-  p.tiles_n = (p.N + kNBN - 1) / kNBN;  // (nor whole tiles of columns: see its rhs descriptor)
+  p.tiles_m = (p.M + kNBM - 1) / kNBM;
+  p.tiles_n = (p.N + kNBN - 1) / kNBN;
   const bool packed = packed_epilogue(p) && !host_has_tail(p);  // (a fused tail goes through the element stores here)
   dim3 grid((unsigned)(p.tiles_m * p.tiles_n), (unsigned)p.split_k);
   if (packed && p.N % 8) nn_kernel<T, BK, STAGES, true, A_TR, B_TR, KTAIL, true><<<grid, dim3(256), 0, s>>>(p);

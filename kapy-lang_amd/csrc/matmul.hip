@@ -498,7 +498,7 @@ int matmul_16bit(const kapy_global *lhs, const kapy_global *rhs, const kapy_glob
   // Roofline path: both operands K-contiguous, 16-byte aligned rows, extents multiples of the tile,
   // and offsets that fit the 32-bit per-lane address arithmetic of the loader.
   bool tn = p.a_sk == 1 && p.b_sk == 1 && vector_bytes(lhs, 1) == 16 && vector_bytes(rhs, 0) == 16 && p.K > 0 &&
-            p.a_sm * 2 * 256 < (int64_t(1) << 31) && p.b_sn * 2 * 256 < (int64_t(1) << 31) && p.a_sm >= 0 && p.b_sn >= 0;
+            p.a_sm * 2 * 256 + (int64_t)p.K * 2 < (int64_t(1) << 31) && p.b_sn * 2 * 256 + (int64_t)p.K * 2 < (int64_t(1) << 31) && p.a_sm >= 0 && p.b_sn >= 0;
   if (tn) {
     const bool free_choice = !c.tile_m && !c.tile_n && !c.tile_k && !c.stages && !c.waves && c.impl_way < KAPY_MFMA_32X32X16_16B;
     for (const TnVariant &v : kTnVariants) {

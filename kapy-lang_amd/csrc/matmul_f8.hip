@@ -492,7 +492,8 @@ int matmul_f8(const kapy_global *a, const kapy_global *b, const float *row_scale
     g.a = (const char *)p.a; g.b = (const char *)p.b; g.acc = nullptr; g.d = p.d;
     g.row_scale = row_scale; g.col_scale = col_scale;
     g.bias = nullptr; g.alpha = 1.0f; g.bias_dtype = KAPY_F32; g.act = -1; g.act_operand = 0.f;
-    g.a_sm = p.a_sm; g.a_sk = 1; g.b_sn = p.b_sn; g.b_sk = 1;
+    g.a_sm = p.M > 1 ? p.a_sm : p.K; g.a_sk = 1;  // (the pitch of a single row, which may be anything, is not stepped over)
+    g.b_sn = p.N > 1 ? p.b_sn : p.K; g.b_sk = 1;
     g.acc_sm = g.acc_sn = 0; g.d_sm = p.d_sm; g.d_sn = p.d_sn;
     g.M = p.M; g.N = p.N; g.K = p.K;
     g.acc_dtype = -1; g.d_dtype = p.d_dtype; g.rz = p.rz; g.tiles_m = g.tiles_n = 0;

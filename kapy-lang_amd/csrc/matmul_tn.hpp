@@ -2,6 +2,7 @@
 // matmul_tn_bf16.hip, matmul_tn_f16.hip and matmul_tn_f8.hip (one translation unit each: they take minutes to compile).
 #pragma once
 #include "matmul_tile.hpp"
+#include "operand_pieces.hpp"
 
 namespace kapy {
 namespace {
@@ -49,21 +50,21 @@ __global__ __launch_bounds__(64 * WM * WN) void tn_kernel(GemmParams p) {
   // Instruction q of an operand fills LDS bytes [q*1024, q*1024+1024); this lane's 16 bytes sit at
   // q*1024 + lane*16, which the (inverse) swizzle maps back to a (row, chunk) of the tile.
   uint32_t a_goff[C::kLoadsAPerWave], b_goff[C::kLoadsBPerWave];
+  // (Rows past an operand's end: the last row again, results nobody stores.  Not in the two-pass ring, which keeps the offset of the
+  // first load only and leaves such rows to the descriptors; the 256-wide builds outside the ring are only given whole tiles.)
+  constexpr bool kRowsReplaced = STAGES == kRing25 ? BK != T::kSliceK : BM <= 128 && BN <= 128;
+  using Pieces = OperandPieces<false, BK, EB>;
 #pragma unroll
   for (int i = 0; i < C::kLoadsAPerWave; ++i) {
     uint32_t row, chunk;
     L::locate((uint32_t)(wave + i * C::kWaves) * 1024u + lane * 16u, row, chunk);
-    // (the 128-wide builds without bounded loads fetch the operand's last row in place of rows past its end: results nobody
-    // stores; the 256-wide ones are only given whole tiles)
-    if constexpr (STAGES != kRing25 && BM <= 128) row = min(row, (uint32_t)max(p.M - 1 - tm * BM, 0));
-    a_goff[i] = (uint32_t)((row * p.a_sm + chunk * (16 / EB)) * EB);
+    a_goff[i] = Pieces::lane(row, chunk * Pieces::kPer, (int32_t)p.a_sm, kRowsReplaced ? p.M - m0 : BM);
   }
 #pragma unroll
   for (int i = 0; i < C::kLoadsBPerWave; ++i) {
     uint32_t row, chunk;
     L::locate((uint32_t)(wave + i * C::kWaves) * 1024u + lane * 16u, row, chunk);
-    if constexpr (STAGES != kRing25 && BN <= 128) row = min(row, (uint32_t)max(p.N - 1 - tn * BN, 0));
-    b_goff[i] = (uint32_t)((row * p.b_sn + chunk * (16 / EB)) * EB);
+    b_goff[i] = Pieces::lane(row, chunk * Pieces::kPer, (int32_t)p.b_sn, kRowsReplaced ? p.N - n0 : BN);
   }
   const char *a_tile = p.a + (int64_t)m0 * p.a_sm * EB;
   const char *b_tile = p.b + (int64_t)n0 * p.b_sn * EB;
@@ -183,9 +184,10 @@ __global__ __launch_bounds__(64 * WM * WN) void tn_kernel(GemmParams p) {
       const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
       return (void *)(((uint64_t)hi << 32) | lo);
     };
-    // The descriptors end where the operands end: in a tile that hangs over the last row of the lhs (M not a multiple
-    // of BM) or of the rhs, the loads of the rows that do not exist are out of range, which the hardware answers with
-    // zeros in LDS instead of a fault.  (An operand with 2 GiB or more behind the tile base has all of the tile's rows.)
+    // The descriptors end where the operands end.  In the two-pass ring, a tile that hangs over the last row of the lhs (M not a
+    // multiple of BM) or of the rhs leaves the rows that do not exist to them: their row offsets are out of range (rows do
+    // not overlap, matmul_tn_f8.hip), which the hardware answers with zeros in LDS instead of a fault.  (An operand with 2 GiB
+    // or more behind the tile base has all of the tile's rows.)
     auto bytes_left = [&](int32_t rows, int64_t pitch) {
       const int64_t left = rows <= 0 ? 0 : ((int64_t)(rows - 1) * pitch + p.K) * EB;
       return (int)(left < 0x7fffffff ? left : 0x7fffffff);

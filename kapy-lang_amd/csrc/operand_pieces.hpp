@@ -37,4 +37,9 @@ struct OperandPieces {
   }
 };
 
+// A loader that forms the offsets of a tile's rows from the first row's cannot replace single rows: it relies on the range check to
+// answer the rows of a K-contiguous operand that do not exist with zeros.  They all start at or behind the operand's end only
+// if rows do not overlap - whether that holds for `rows` rows cut into tiles of `tile`.
+constexpr bool rows_end_at_descriptor(int64_t rows, int64_t pitch, int64_t k, int tile) { return rows % tile == 0 || pitch >= k; }
+
 }  // namespace kapy

@@ -40,6 +40,24 @@ static void walk(int width, int left, int k, int64_t ld) {
   }
 }
 
+// A loader that leaves rows that do not exist to the range check: wherever rows_end_at_descriptor allows it, every piece of such a
+// row must be out of range, whether or not the check counts the scalar part.
+template <int BK, int EB>
+static void walk_rows(int width, int rows, int k, int64_t ld) {
+  using P = kapy::OperandPieces<false, BK, EB>;
+  if (!kapy::rows_end_at_descriptor(rows, ld, k, width)) return;
+  const int left = rows % width ? rows % width : width, tiles = (k + BK - 1) / BK;
+  const int64_t bytes = P::bytes(k, ld, left);
+  for (int j = 0; j < tiles; ++j)
+    for (int line = left; line < width; ++line)
+      for (int first = 0; first < BK; first += 16 / EB, ++checked) {
+        const int64_t lane = P::lane((uint32_t)line, (uint32_t)first, (int32_t)ld, width), scalar = P::tile(j, tiles, (int32_t)ld);
+        if (lane >= bytes - scalar && lane >= bytes && scalar <= bytes) continue;
+        std::printf("a row that does not exist is in range: %d rows in tiles of %d, K %d, pitch %lld: K-tile %d row %d position %d\n", rows, width, k, (long long)ld, j, line, first);
+        std::exit(1);
+      }
+}
+
 template <int BK, int EB>
 static void walk_all(int width) {
   const int lefts[] = {1, 2, 7, 8, 9, 31, 32, 33, 40, 96, 104, 120, 127, 128, 129, 136, 232, 248, 255, 256, 300};
@@ -49,6 +67,8 @@ static void walk_all(int width) {
   for (int left : lefts) {
     for (int k : ks)
       for (int64_t ld : {(int64_t)k, (int64_t)k + per, (int64_t)4 * k, (int64_t)per, (int64_t)0}) walk<false, BK, EB>(width, left, k, ld);  // (rows may overlap, or all be one row)
+    for (int k : ks)
+      for (int64_t ld : {(int64_t)k, (int64_t)k + per, (int64_t)4 * k, (int64_t)per, (int64_t)k - per, (int64_t)0}) walk_rows<BK, EB>(width, left, k, ld);
     if (EB != 2) continue;
     for (int k : odd_ks)  // (a line that ends inside a piece: the pitch is whole pieces)
       for (int64_t ld : {(int64_t)(k + per - 1) / per * per, (int64_t)(k + 5 * per) / per * per}) walk<false, BK, EB>(width, left, k, ld);

@@ -588,8 +588,10 @@ bool packed_epilogue(const GemmParams &p) {
   const int64_t eb = p.d_dtype == KAPY_F32 ? 4 : 2, ab = p.acc_dtype == KAPY_F32 ? 4 : 2;
   // an accumulator input: f16 or f32, row-major with 16-byte aligned rows, and neither scales nor a fused tail beside it
   const bool acc_ok = p.acc_dtype < 0 || ((p.acc_dtype == KAPY_F16 || p.acc_dtype == KAPY_F32) && p.acc_sn == 1 && ((uintptr_t)p.acc & 15) == 0 &&
-                                          (p.acc_sm * ab) % 16 == 0 && p.acc_sm * ab * 256 < (int64_t(1) << 31) && !p.row_scale && !host_has_tail(p));
-  return (p.d_dtype == KAPY_F16 || p.d_dtype == KAPY_BF16 || p.d_dtype == KAPY_F32) && p.d_sn == 1 && acc_ok && (!p.rz || p.d_dtype == KAPY_F32) &&
+                                          p.acc_sm >= 0 && (p.acc_sm * ab) % 16 == 0 && p.acc_sm * ab * 256 < (int64_t(1) << 31) && !p.row_scale && !host_has_tail(p));
+  // (the descriptor of a wave's part of the result ends with the last row: it keeps rows that do not exist out only if rows lie one
+  // behind the other, so a single row of any pitch goes element by element, and rows in reverse order do)
+  return (p.d_dtype == KAPY_F16 || p.d_dtype == KAPY_BF16 || p.d_dtype == KAPY_F32) && p.d_sn == 1 && p.d_sm >= p.N && acc_ok && (!p.rz || p.d_dtype == KAPY_F32) &&
          ((uintptr_t)p.d & 15) == 0 && (p.d_sm * eb) % 16 == 0 && p.d_sm * eb * 256 < (int64_t(1) << 31) &&  // (a wave's rows are addressed with 32-bit offsets)
          (!p.row_scale || ((uintptr_t)p.col_scale & 15) == 0);
 }

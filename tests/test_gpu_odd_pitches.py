@@ -60,3 +60,27 @@ def test_f8_rows_that_overlap(ko, M, N, K):
 def test_f8_single_row_of_any_pitch(ko, N, K):
     for pitch in (1, 3, 16):
         _check(ko, kh.F8E4M3, 1, N, K, pitch, K, kh.F32, 1e-4, 85)
+
+
+@pytest.mark.parametrize("out", [kh.F32, kh.F16])
+@pytest.mark.parametrize("M,N,K,b_rm", [(1, 136, 128, False), (1, 264, 192, True), (40, 136, 64, False), (300, 264, 128, True), (300, 264, 128, False), (257, 520, 72, True)])
+def test_results_of_any_row_pitch(ko, out, M, N, K, b_rm):
+    """A single result row of any pitch, and result rows in reverse order: stored where they belong and nothing else touched."""
+    a, b = ko.fill_normal(M * K, kh.F16, 86, 0, 0.0, 0.5), ko.fill_normal(K * N, kh.F16, 86, 1, 0.0, 0.5)
+    b_str = (N, 1) if b_rm else (1, K)
+    want = np.zeros(M * N, np.float32 if out == kh.F32 else np.uint16)
+    assert ko.lib().ko_matmul(C.byref(ko.mk_global(a, M, K, K, 1, kh.F16)), C.byref(ko.mk_global(b, K, N, *b_str, kh.F16)), None,
+                              C.byref(ko.mk_global(want, M, N, N, 1, out)), kh.RN) == 0
+    da, db = to_dev(a), to_dev(b)
+    for pitch in ((0, 8, -N) if M == 1 else (-N, -N - 8)):
+        span = (M - 1) * -pitch if M > 1 else 0
+        dd = dev_zeros(span + N + 512, kh.DTYPE_BYTES[out], fill=0x1234)
+        kh.matmul(dglobal(da, M, K, K, 1, kh.F16), dglobal(db, K, N, *b_str, kh.F16), dglobal(dd, M, N, pitch, 1, out, dynamic_offset=span + 256))
+        sync()
+        got = to_host(dd, want.dtype)
+        at = span + 256 + np.arange(M)[:, None] * pitch + np.arange(N)
+        g, w = ko.decode(np.ascontiguousarray(got[at].ravel()), out), ko.decode(want, out)
+        assert np.all(np.isfinite(g)) and np.linalg.norm(g - w) <= (1e-5 if out == kh.F32 else 1e-3) * np.linalg.norm(w), pitch
+        rest = np.ones(got.size, bool)
+        rest[at.ravel()] = False
+        assert np.all(got[rest].view(np.uint32 if out == kh.F32 else np.uint16) == 0x1234), pitch

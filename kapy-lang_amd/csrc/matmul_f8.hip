@@ -478,7 +478,9 @@ int matmul_f8(const kapy_global *a, const kapy_global *b, const float *row_scale
   if (p.M == 0 || p.N == 0) return KAPY_OK;
   // K-contiguous operands with 16-byte aligned rows of whole 16-byte pieces: what the tiled kernel needs (its ring builds take
   // a partial last K-tile); the streaming kernels below need whole 128-byte K steps
-  const bool k_pieces = p.a_sk == 1 && p.b_sk == 1 && vector_bytes(a, 1) == 16 && vector_bytes(b, 0) == 16 && p.K % 16 == 0 && p.K > 0;
+  // (and unsigned 32-bit row offsets: rows in reverse order go to the general kernels)
+  const bool k_pieces = p.a_sk == 1 && p.b_sk == 1 && vector_bytes(a, 1) == 16 && vector_bytes(b, 0) == 16 && p.K % 16 == 0 && p.K > 0 &&
+                        (p.M == 1 || p.a_sm >= 0) && (p.N == 1 || p.b_sn >= 0);
   const bool k_contig = k_pieces && p.K % 128 == 0;
   // Many rows: the tiled LDS-direct kernel (MFMA-bound).  Few rows: the skinny kernel (HBM-bound).
   // With a workspace the tiled kernel can split K over several workgroups per tile, which fills the device at few rows too.

@@ -1,6 +1,6 @@
 """Matrix products on operands whose rows do not lie one behind the other: rows that overlap (a pitch below the row's length), a single
-row whose pitch is anything.  A tile over the edge of such an operand cannot rely on its pitch to tell rows that exist from rows
-that do not; the sizes are tiles that hang over the rows, whole and partial last K-tiles.  Against the oracle."""
+row whose pitch is anything, rows in reverse order.  A tile over the edge of such an operand cannot rely on its pitch to tell rows
+that exist from rows that do not; the sizes are tiles that hang over the rows, whole and partial last K-tiles.  Against the oracle."""
 import ctypes as C
 
 import numpy as np
@@ -19,12 +19,13 @@ def _check(ko, dt, M, N, K, a_pitch, b_pitch, out, tol, seed, **cfg):
         codes = lambda n: rng.integers(0x20, 0x50, size=n).astype(np.uint8) | (rng.integers(0, 2, size=n).astype(np.uint8) << 7)  # noqa: E731
     else:
         codes = lambda n: ko.fill_normal(n, dt, seed, n % 7, 0.0, 0.5)  # noqa: E731
-    a, b = codes((M - 1) * a_pitch + K), codes((N - 1) * b_pitch + K)
+    a, b = codes((M - 1) * abs(a_pitch) + K), codes((N - 1) * abs(b_pitch) + K)
+    a0, b0 = (M - 1) * max(-a_pitch, 0), (N - 1) * max(-b_pitch, 0)   # element (0, 0): the last row's place where rows run backwards
     want = np.zeros(M * N, np.float32 if out == kh.F32 else np.uint16)
-    assert ko.lib().ko_matmul(C.byref(ko.mk_global(a, M, K, a_pitch, 1, dt)), C.byref(ko.mk_global(b, K, N, 1, b_pitch, dt)), None,
+    assert ko.lib().ko_matmul(C.byref(ko.mk_global(a, M, K, a_pitch, 1, dt, a0)), C.byref(ko.mk_global(b, K, N, 1, b_pitch, dt, b0)), None,
                               C.byref(ko.mk_global(want, M, N, N, 1, out)), kh.RN) == 0
     da, db, dd = to_dev(a), to_dev(b), dev_zeros(M * N + 64, kh.DTYPE_BYTES[out], fill=0x1234)
-    kh.matmul(dglobal(da, M, K, a_pitch, 1, dt), dglobal(db, K, N, 1, b_pitch, dt), dglobal(dd, M, N, N, 1, out), **cfg)
+    kh.matmul(dglobal(da, M, K, a_pitch, 1, dt, a0), dglobal(db, K, N, 1, b_pitch, dt, b0), dglobal(dd, M, N, N, 1, out), **cfg)
     sync()
     got = to_host(dd, want.dtype)
     assert np.all(got[M * N:].view(np.uint32 if out == kh.F32 else np.uint16) == 0x1234)
@@ -60,6 +61,13 @@ def test_f8_rows_that_overlap(ko, M, N, K):
 def test_f8_single_row_of_any_pitch(ko, N, K):
     for pitch in (1, 3, 16):
         _check(ko, kh.F8E4M3, 1, N, K, pitch, K, kh.F32, 1e-4, 85)
+
+
+@pytest.mark.parametrize("dt,M,N,K", [(kh.F8E4M3, 16, 128, 512), (kh.F8E4M3, 48, 136, 512), (kh.F8E4M3, 200, 136, 256), (kh.F8E4M3, 300, 520, 272), (kh.F8E4M3, 5, 48, 128),
+                                      (kh.BF16, 200, 136, 128), (kh.F16, 300, 264, 72)])
+def test_operand_rows_in_reverse_order(ko, dt, M, N, K):
+    for a_pitch, b_pitch in ((-K, K), (K, -K - 16), (-K, -K)):
+        _check(ko, dt, M, N, K, a_pitch, b_pitch, kh.F32, 1e-4 if kh.DTYPE_BYTES[dt] == 1 else 1e-5, 87)
 
 
 @pytest.mark.parametrize("out", [kh.F32, kh.F16])

@@ -43,6 +43,7 @@
 static __device__ __align__(256) unsigned char scratch[kapy::kSplitCounterBytes + (16 << 20)];
 
 #include "matmul_tile.hpp"
+#include "wide_rule.hpp"
 
 namespace kapy {
 namespace {
@@ -326,19 +327,6 @@ bool wide_serves(const GemmParams &p, int bn, bool a_tr, bool b_tr) {
   return a_fits && b_fits && ((int64_t)(p.M + 255) / 256) * ((p.N + bn - 1) / bn) < limit;
 }
 
-// Rounds of tiles over the CUs decide: a 256 x 128 tile takes 0.54 of a 256 x 256 tile's time (the larger one reads fewer LDS bytes per
-// flop), so the narrower tile wins where the wide one leaves CUs idle in its only or its last round.  Not where 128 x 128 tiles
-// fit the CUs in one round: they use twice as many CUs.  Measured (us: 128 x 128, 256 x 128, 256 x 256; bf16 K-contiguous unless said):
-//   2048 x 4096 x 4096   59.2   53.2   69.5     1100 x 4096 x 4096   43.5   41.8   63.8     1973 x 2560 x 3072, row-major rhs   45.2   36.9   -
-//   4096 x 5120 x 2048   76.4   77.7   83.4     3333 x 3328 x 2048   49.0   50.6   41.7     (256 x 256 in one round: kept)
-//   500 x 8192 x 4096    36.6   40.9   66.3     (128 x 128 in one round: kept)
-//   fp8 1000 x 8192 x 8192   59.3   54.1   74.2     fp8 2816 x 7168 x 4096   78.5   77.0   85.5     fp8 1500 x 8192 x 8192   90.7   90.5   80.5
-bool prefer_wide128(int64_t m, int64_t n) {
-  const int64_t cus = device_cus();
-  auto rounds = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm * ((n + bn - 1) / bn) + cus - 1) / cus; };
-  return rounds(128, 128) > 1 && rounds(256, 128) * 108 < rounds(256, 256) * 200;
-}
-
 // Implemented in matmul_f8.hip.
 int matmul_f8(const kapy_global *a, const kapy_global *b, const float *row_scale, const float *col_scale, const kapy_global *acc,
               const kapy_global *result, const kapy_matmul_cfg *cfg, hipStream_t s);
@@ -420,7 +408,7 @@ int matmul_16bit(const kapy_global *lhs, const kapy_global *rhs, const kapy_glob
   const bool wide_asked = c.tile_m == 256 && c.tile_n == 128 && (!c.tile_k || c.tile_k == 64) && !c.stages && (!c.waves || c.waves == 4) && c.split_k <= 1 && c.impl_way != KAPY_MFMA_32X32X16_16B;
   int wide_bn = 0;
   if (wide_form && (wide_free || wide_asked)) {
-    if ((wide_asked || prefer_wide128(p.M, p.N)) && wide_serves(p, 128, column_lhs, row_rhs)) wide_bn = 128;
+    if ((wide_asked || wide128_wins(p.M, p.N, p.K, row_rhs ? 0 : 512, device_cus())) && wide_serves(p, 128, column_lhs, row_rhs)) wide_bn = 128;
     // (KAPY_NN256=0 in the environment: never the 256 x 256 form; KAPY_NN256_FROM: the least number of its tiles per 100 CUs, for
     // measurements)
     static const bool wide256 = !(getenv("KAPY_NN256") && getenv("KAPY_NN256")[0] == '0');
@@ -510,9 +498,8 @@ int matmul_16bit(const kapy_global *lhs, const kapy_global *rhs, const kapy_glob
       const bool whole_tiles = p.M % v.bm == 0 && p.N % v.bn == 0;
       const bool whole_k = p.K % v.bk == 0;  // the ring variants also take a partial last K-tile of whole 16-byte chunks
       if ((!whole_k && (v.stages != kRing25 || p.K % 8)) || (!whole_tiles && v.stages != kRing25)) continue;
-      // with a free choice, a 256x256 tiling with fewer than 0.55 tiles per CU yields to 128x128 (measured: 144 large tiles on
-      // 256 CUs beat 576 small ones - 3072^3: 1009 against 899 TFLOP/s - 128 do not)
-      if (free_choice && v.bm == 256 && (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256) * 100 < (int64_t)device_cus() * 55) continue;
+      // with a free choice, a 256x256 tiling of too few tiles yields to 128x128
+      if (free_choice && v.bm == 256 && !enough_256_tiles(p.M, p.N, device_cus())) continue;
       // an explicit split of K is a request for a variant that can split: with a free tile choice the others are passed over
       // (plan_split_k then honours the split or says why it cannot)
       if (c.split_k > 1 && !c.tile_m && !(v.bm == 128 && v.stages == kRing25)) continue;

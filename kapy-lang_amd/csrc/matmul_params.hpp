@@ -75,7 +75,4 @@ int launch_wide128_f16(const GemmParams &p, bool a_tr, bool b_tr, hipStream_t s)
 // 256 x 128 x 128 tiles on fp8 operands, both K-contiguous, K in whole tiles.
 int launch_wide128_f8(const GemmParams &p, int lhs_fmt, int rhs_fmt, hipStream_t s);
 
-// Whether a result of m x n is better cut into 256 x 128 tiles than into the 256 x 256 or 128 x 128 ones.
-bool prefer_wide128(int64_t m, int64_t n);
-
 }  // namespace kapy

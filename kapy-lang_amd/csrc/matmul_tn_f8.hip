@@ -1,5 +1,6 @@
 // matmul_tn_f8.hip — the tiled kernel on fp8 operands.
 #include "matmul_tn.hpp"
+#include "wide_rule.hpp"
 
 namespace kapy {
 namespace {
@@ -24,13 +25,13 @@ int matmul_f8_tiled(const GemmParams &p, int lhs_fmt, int rhs_fmt, int want_tile
   if (p.K % 16 == 0 && p.K >= 128 && p.M >= 1 && p.N >= 128) {
     // (want_tile: 0 = the library's choice, 128 or 256 = the caller's, kapy_matmul_cfg.tile_m; kWideTile: 256 x 128)
     // (measured at N = K = 8192: 192 of the large tiles on 256 CUs already beat 768 of the small ones, 128 do not)
-    if ((want_tile == kWideTile || (want_tile == 0 && p.split_k <= 1 && prefer_wide128(p.M, p.N))) && p.K % 128 == 0 && p.N % 8 == 0 && packed_epilogue(p))
+    if ((want_tile == kWideTile || (want_tile == 0 && p.split_k <= 1 && wide128_wins(p.M, p.N, p.K, 2048, device_cus()))) && p.K % 128 == 0 && p.N % 8 == 0 && packed_epilogue(p))
       return launch_wide128_f8(p, lhs_fmt, rhs_fmt, s);
     // Overlapping rows (a pitch below K) in a tile over an edge: the ring builds would read rows that do not exist from behind the
     // operand; the four-stage build replaces them.
     if (!rows_end_at_descriptor(p.M, p.a_sm, p.K, 256) || !rows_end_at_descriptor(p.N, p.b_sn, p.K, 256))
       return p.K % 128 == 0 ? launch_f8<F8, 128, 128, 128, 2, 2, 4>(p, lhs_fmt, rhs_fmt, s) : KAPY_ERR_UNSUPPORTED;
-    if (want_tile == 256 || (want_tile == 0 && (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256) * 100 >= (int64_t)device_cus() * 55))
+    if (want_tile == 256 || (want_tile == 0 && enough_256_tiles(p.M, p.N, device_cus())))
       return launch_f8<F8M16, 256, 256, 128, 2, 2, kRing25>(p, lhs_fmt, rhs_fmt, s);
     // At most one 128 x 128 tile per CU and K not split: the ring build's 2.5 tiles of loads in flight are sized for two
     // workgroups per CU, and one alone waits for them (N = K = 8192, 161 .. 512 rows: 50 us whatever M is).  The four-stage

@@ -32,4 +32,13 @@ constexpr bool wide128_wins(int64_t m, int64_t n, int64_t k, int64_t k_from, int
   return k >= k_from || enough_256_tiles(m, n, cus);
 }
 
+// The tile of an fp8 product: what the caller asked for (kapy_matmul_cfg: 0, 128 or 256 rows; any other request is the library's
+// choice), 256 x 128 where that was asked for or wins and the kernel serves the problem.
+enum F8Tile { kTileFree, kTile128, kTile256, kTileWide };
+constexpr F8Tile f8_tile(int tile_m, int tile_n, bool wide_serves, bool wide_wins) {
+  if (tile_m == 256) return tile_n == 128 && wide_serves ? kTileWide : kTile256;
+  if (tile_m == 128) return kTile128;
+  return wide_serves && wide_wins ? kTileWide : kTileFree;
+}
+
 }  // namespace kapy

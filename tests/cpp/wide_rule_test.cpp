@@ -25,6 +25,20 @@ int main() {
       std::printf("%ld x %ld, K %ld (from %ld): 256 x 128 tiles should be %s\n", r.m, r.n, r.k, r.k_from, r.wide ? "chosen" : "passed over");
       ++bad;
     }
+  // fp8 tiles: 256 x 128 asked for where it does not serve is 256 x 256, as any request of 256 rows is
+  using namespace kapy;
+  const struct {
+    int m, n;
+    bool serves, wins;
+    F8Tile want;
+  } tiles[] = {{256, 128, true, false, kTileWide}, {256, 128, false, false, kTile256}, {256, 128, false, true, kTile256}, {256, 256, true, true, kTile256},
+               {256, 0, true, true, kTile256}, {128, 128, true, true, kTile128}, {128, 0, true, true, kTile128}, {0, 0, true, true, kTileWide},
+               {0, 128, true, true, kTileWide}, {0, 0, false, true, kTileFree}, {0, 0, true, false, kTileFree}, {64, 64, true, false, kTileFree}};
+  for (const auto &t : tiles)
+    if (f8_tile(t.m, t.n, t.serves, t.wins) != t.want) {
+      std::printf("fp8 tile %d x %d (serves %d, wins %d): %d instead of %d\n", t.m, t.n, t.serves, t.wins, f8_tile(t.m, t.n, t.serves, t.wins), t.want);
+      ++bad;
+    }
   if (!bad) std::printf("wide rule ok\n");
   return bad != 0;
 }

@@ -273,6 +273,18 @@ int operand_mode(int64_t s_row, int64_t s_k) { return s_k == 1 ? kKContig : (s_r
 
 int64_t split_workspace_bytes(int64_t tiles, int split) { return kSplitCounterBytes + tiles * split * (128 * 128 * 4); }
 
+// Whether K falls into `sp` parts of whole K-tiles whose partial sums fit the workspace.
+bool split_fits(const GemmParams &p, const kapy_matmul_cfg &c, int tile_k, int sp) {
+  const int64_t tiles = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128);
+  return p.K % (tile_k * sp) == 0 && tiles <= kSplitCounterBytes / 4 && split_workspace_bytes(tiles, sp) <= c.workspace_bytes && ((uintptr_t)c.workspace & 15) == 0;
+}
+bool split_is_valid(int split) { return split >= 0 && split <= kMaxSplitK && !(split & (split - 1)); }
+
+// Whether plan_split_k honours cfg.split_k.
+bool split_is_honoured(const GemmParams &p, const kapy_matmul_cfg &c, int tile_k) {
+  return c.split_k == 0 || c.split_k == 1 || (split_is_valid(c.split_k) && c.workspace && split_fits(p, c, tile_k, c.split_k));
+}
+
 }  // namespace
 
 // Decides whether the 128 x 128 tiled kernels split K for this problem and points the parameters at the workspace.
@@ -283,7 +295,7 @@ int plan_split_k(GemmParams &p, const kapy_matmul_cfg &c, int tile_k) {
   p.split_k = 1;
   p.partial = nullptr;
   p.counters = nullptr;
-  if (c.split_k < 0 || c.split_k > kMaxSplitK || (c.split_k & (c.split_k - 1)))
+  if (!split_is_valid(c.split_k))
     return fail(KAPY_ERR_INVALID, "matmul: split_k must be 0 (library's choice) or a power of two up to %d, not %d", kMaxSplitK, c.split_k);
   if (c.split_k == 1) return KAPY_OK;
   if (!c.workspace) {
@@ -291,20 +303,16 @@ int plan_split_k(GemmParams &p, const kapy_matmul_cfg &c, int tile_k) {
     return KAPY_OK;
   }
   const int64_t tiles = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128);
-  auto fits = [&](int sp) {
-    return p.K % (tile_k * sp) == 0 && tiles <= kSplitCounterBytes / 4 && split_workspace_bytes(tiles, sp) <= c.workspace_bytes &&
-           ((uintptr_t)c.workspace & 15) == 0;
-  };
   int split = 1;
   if (c.split_k > 1) {
-    if (!fits(c.split_k))
+    if (!split_fits(p, c, tile_k, c.split_k))
       return fail(KAPY_ERR_UNSUPPORTED, "matmul: cannot split K = %d into %d parts of whole %d-wide K-tiles with a 16-byte aligned workspace of %lld bytes (%lld needed)",
                   p.K, c.split_k, tile_k, (long long)c.workspace_bytes, (long long)split_workspace_bytes(tiles, c.split_k));
     split = c.split_k;
   } else if (tiles * 2 <= device_cus()) {
     // (meeting in the workspace costs about 10 us: parts shorter than 16 K-tiles do not earn it back)
     for (int sp = 2; sp <= kMaxSplitK && tiles * sp <= device_cus(); sp *= 2)
-      if (fits(sp) && p.K / (tile_k * sp) >= 16) split = sp;
+      if (split_fits(p, c, tile_k, sp) && p.K / (tile_k * sp) >= 16) split = sp;
   }
   if (split > 1) {
     p.split_k = split;
@@ -406,14 +414,17 @@ int matmul_16bit(const kapy_global *lhs, const kapy_global *rhs, const kapy_glob
   const bool wide_form = (row_lhs && (row_rhs || column_rhs)) || (column_lhs && row_rhs);
   const bool wide_free = !c.tile_m && !c.tile_n && !c.tile_k && !c.stages && !c.waves && c.split_k <= 1 && c.impl_way != KAPY_MFMA_32X32X16_16B && !(column_rhs && c.impl_way >= KAPY_MFMA_32X32X16_16B);
   const bool wide_asked = c.tile_m == 256 && c.tile_n == 128 && (!c.tile_k || c.tile_k == 64) && !c.stages && (!c.waves || c.waves == 4) && c.split_k <= 1 && c.impl_way != KAPY_MFMA_32X32X16_16B;
+  // (a split that is no split at all is left to the kernels below, which refuse it; two row-major operands on 256 x 256 tiles never
+  // looked at it)
+  const bool split_said = c.split_k >= 0;
   int wide_bn = 0;
   if (wide_form && (wide_free || wide_asked)) {
-    if ((wide_asked || wide128_wins(p.M, p.N, p.K, row_rhs ? 0 : 512, device_cus())) && wide_serves(p, 128, column_lhs, row_rhs)) wide_bn = 128;
+    if (split_said && (wide_asked || wide128_wins(p.M, p.N, p.K, row_rhs ? 0 : 512, device_cus())) && wide_serves(p, 128, column_lhs, row_rhs)) wide_bn = 128;
     // (KAPY_NN256=0 in the environment: never the 256 x 256 form; KAPY_NN256_FROM: the least number of its tiles per 100 CUs, for
     // measurements)
     static const bool wide256 = !(getenv("KAPY_NN256") && getenv("KAPY_NN256")[0] == '0');
     static const int wide256_from_pct = getenv("KAPY_NN256_FROM") ? atoi(getenv("KAPY_NN256_FROM")) : 55;
-    if (!wide_bn && wide_free && wide256 && row_rhs && wide_serves(p, 256, column_lhs, row_rhs) &&
+    if (!wide_bn && wide_free && (split_said || row_lhs) && wide256 && row_rhs && wide_serves(p, 256, column_lhs, row_rhs) &&
         (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256) * 100 >= (int64_t)device_cus() * wide256_from_pct)
       wide_bn = 256;
   }
@@ -545,8 +556,12 @@ int matmul_16bit(const kapy_global *lhs, const kapy_global *rhs, const kapy_glob
     };
     static const NnVariant kNn[] = {{64, 4}, {64, 3}, {32, 4}};
     const int form = !a_tr ? (b_tr ? 0 : 3) : (b_tr ? 1 : 2);
+    // A split that cannot be honoured is refused, except where lines end inside the tiles' pieces (a row-major result's in N, a
+    // column-major lhs's in M): such calls keep going to the general kernel, which does not split.
+    const bool any_split = p.N % 8 || (a_tr && p.M % kNBM);
     for (const NnVariant &v : kNn) {
       if ((c.tile_k && c.tile_k != v.bk) || (c.stages && c.stages != v.stages) || p.K % v.bk) continue;
+      if (any_split && !split_is_honoured(p, c, v.bk)) break;
       rc = plan_split_k(p, c, v.bk);
       if (rc) return rc;
       return launch_nn_config(p, bf16, form, v.bk, v.stages, false, s);

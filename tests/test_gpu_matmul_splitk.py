@@ -175,3 +175,35 @@ def test_an_explicit_split_with_a_free_tile_choice_is_honoured(ko):
         kh.matmul(ga, gb, dglobal(split, M, N, N, 1, dt), split_k=2, workspace=(ws.data_ptr(), 16384 + 4096))
     assert e.value.status == kh.ERR_UNSUPPORTED
 
+
+
+@pytest.mark.parametrize("M,N,K,b_row_major", [(1100, 4096, 512, False), (1100, 4096, 512, True), (264, 256, 128, True)])
+def test_a_split_that_is_none_is_refused_whatever_the_tile(ko, M, N, K, b_row_major):
+    """Shapes whose tile the library picks by its rule for 256 x 128 tiles, and that tile by name."""
+    dt = kh.BF16
+    da, db, dd = dev_zeros(M * K, 2), dev_zeros(K * N, 2), dev_zeros(M * N, 2)
+    ga, gb, gd = dglobal(da, M, K, K, 1, dt), dglobal(db, K, N, *((N, 1) if b_row_major else (1, K)), dt), dglobal(dd, M, N, N, 1, dt)
+    with pytest.raises(kh.KapyError) as e:
+        kh.matmul(ga, gb, gd, split_k=-1)
+    assert e.value.status == kh.ERR_INVALID
+    with pytest.raises(kh.KapyError) as e:
+        kh.matmul(ga, gb, gd, split_k=-1, tile=(256, 128, 64))
+    assert e.value.status == kh.ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("M,N,K,a_row_major", [(136, 131, 256, True), (136, 131, 320, True), (200, 264, 128, False)])
+def test_lines_that_end_inside_the_tiles_take_a_split_that_cannot_be_honoured(ko, M, N, K, a_row_major):
+    """N no multiple of 8, or M no multiple of 128 for a column-major lhs: any split_k is accepted, and one that cannot be honoured (no
+    workspace, no power of two, parts of broken K-tiles) leaves K whole."""
+    dt, pitch = kh.F16, (N + 7) // 8 * 8
+    a, b = ko.fill_uniform(M * K, dt, 71, 0), ko.fill_uniform(K * pitch, dt, 71, 1)
+    a_str = (K, 1) if a_row_major else (1, M)
+    want = np.zeros(M * N, np.float32)
+    assert ko.lib().ko_matmul(C.byref(ko.mk_global(a, M, K, *a_str, dt)), C.byref(ko.mk_global(b, K, N, pitch, 1, dt)), None,
+                              C.byref(ko.mk_global(want, M, N, N, 1, kh.F32)), kh.RN) == 0
+    da, db = to_dev(a), to_dev(b)
+    for kw in (dict(split_k=2), dict(split_k=-1), dict(split_k=3), dict(split_k=8, workspace=_workspace(M, N))):
+        dd = dev_zeros(M * N, 4)
+        kh.matmul(dglobal(da, M, K, *a_str, dt), dglobal(db, K, N, pitch, 1, dt), dglobal(dd, M, N, N, 1, kh.F32), **kw)
+        sync()
+        assert _frob(ko, to_host(dd, np.float32), want, kh.F32) <= 1e-5, kw

@@ -326,3 +326,22 @@ def test_device_entry_points_fail_loudly_without_a_gpu():
     assert st == kh.ERR_HIP
     st, msg = _status(kh.elementwise, kh.gelu_program(), [x, _g(m=1, n=16)], x, stream=NULL)
     assert st == kh.ERR_HIP
+
+
+@pytest.mark.parametrize("missing", ["_cuda_getCurrentRawStream", "_cuda_getDevice", None])
+def test_current_stream_without_torchs_private_functions(monkeypatch, missing):
+    """The raw handle is a shortcut: a torch that lacks either function, or has not initialised the GPU, is asked for its Stream object."""
+    import torch
+
+    class Stream:
+        cuda_stream = 0x5678
+
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 0x1000 + device, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 3, raising=False)
+    if missing:
+        monkeypatch.delattr(torch._C, missing)
+    assert kh.current_stream().value == (0x5678 if missing else 0x1003)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: False)
+    assert kh.current_stream().value == 0x5678

@@ -5,8 +5,9 @@
 
 A step is one pass of the hot path over one batch of synthetic input, inputs resident in HBM.
 The headline workload (the configuration the headline metric is quoted on) is the fused elementwise
-y = GELU_tanh(x*0.5 + bias) on fp16 8192x8192; the JSON line also carries every other benchmark
-configuration under "other_workloads", each with its own roofline.  One JSON line on stdout.
+y = GELU_tanh(x*0.5 + bias) on fp16 8192x8192.  One short JSON line on stdout: the headline and, under
+config.configs, the figures of every benchmark configuration.  The full records of the other workloads, each with
+its own roofline, go to stderr before it, a JSON line each.
 
 Inputs are the ones each configuration states, generated on the host by the seeded counter-based generators of
 the CPU checker (fp64, rounded once to the storage type) and uploaded: the GPU and the checker see the same bytes.
@@ -1134,10 +1135,7 @@ def stats_summary(stats_csv):
 
 def ceilings_summary(bench_json):
     """The tracked summary of the probe kernels' figures from the JSON line of `bench.py --workload ceilings --no-others`."""
-    line = json.loads(open(bench_json).read().strip().split("\n")[-1])
-    res = next((r for r in [line.get("config", {})] + line.get("other_workloads", []) if "mfma" in r), None)
-    if res is None:
-        res = line
+    res = json.loads(open(bench_json).read().strip().split("\n")[-1])
     out = ["Device ceilings measured by the probe library's kernels (libkapy_probe.so) and the tiled GEMMs' fixed cost per launch, one MI355X (gfx950)", "",
            "commands (from the repository root):",
            "  python3 bench.py --no-cpu --no-others --workload ceilings > gpurun_out/ceilings.json",
@@ -1164,6 +1162,34 @@ def ceilings_summary(bench_json):
         if key in res:
             out.append("%-40s %s" % (key, res[key]))
     print("\n".join(out))
+
+
+def summary_line(args, main_res, by_name):
+    """The one line on stdout: the headline workload, and of every benchmark configuration that was measured its figures.  Short (a log
+    that keeps only its last few KB keeps it whole); the other workloads' full records go to stderr, a line each."""
+    configs = {}
+    for cfg, name in (("C1", "gemm_f16"), ("C2", "gelu"), ("C3a", "transpose"), ("C3b", "permute"), ("C4", "gemm_bf16"), ("C5_M16", "f8_m16"), ("C5_M4096", "f8_m4096")):
+        r = by_name.get(name)
+        if r is None:
+            continue
+        if "roofline" not in r:
+            configs[cfg] = {"checked": False, "error": r.get("error", "not run")[:200]}
+            continue
+        configs[cfg] = {"value": round(r["value"], 2), "unit": r["unit"], "kernel_ms": round(r["kernel_ms"], 4), "bound": r["roofline"]["bound"],
+                        "frac": r["roofline"]["frac"], "checked": r["checked"], "kernel": r["kernel"],
+                        "cpu_baseline": (r.get("cpu_baseline") or {}).get("value"), "cpu_unit": (r.get("cpu_baseline") or {}).get("unit")}
+    return {
+        "metric": "GEMM TFLOP/s + % MFMA peak; elementwise/transpose GB/s + % HBM peak (1 GPU)",
+        "value": round(main_res["value"], 2), "unit": main_res["unit"], "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
+        "ms_per_step": round(main_res["ms_per_step"], 4), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
+        "dtype": main_res["dtype"], "data": "synthetic",
+        "config": {"workload": main_res["workload"], "kernel": main_res["kernel"], "kernel_ms": round(main_res["kernel_ms"], 4),
+                   "inputs": main_res["inputs"], "checked": main_res["checked"], "check": main_res["check"],
+                   "buffers": "4 rotating sets (1 GiB) so reads miss the Infinity Cache" if main_res["unit"] == "GB/s" else "single set",
+                   "configs": configs, **({"programs": main_res["programs"]} if "programs" in main_res else {})},
+        "roofline": main_res["roofline"],
+        "cpu_baseline": main_res.get("cpu_baseline"),
+    }
 
 
 def main():
@@ -1260,35 +1286,9 @@ def main():
                 r["ms_per_step"] = round(r["ms_per_step"], 4)
                 r["kernel_ms"] = round(r["kernel_ms"], 4)
             others.append(r)
-    # every benchmark configuration in one compact block inside "config" (a key that records of this line keep), and the long
-    # tables first in the line, so that its end - what a truncated log keeps - holds the configurations and the headline
-    by_name = dict([(args.workload, main_res)] + [(n, r) for n, r in zip(other_names, others)])
-    configs = {}
-    for cfg, name in (("C1", "gemm_f16"), ("C2", "gelu"), ("C3a", "transpose"), ("C3b", "permute"), ("C4", "gemm_bf16"), ("C5_M16", "f8_m16"), ("C5_M4096", "f8_m4096")):
-        r = by_name.get(name)
-        if r is None:
-            continue
-        if "roofline" not in r:
-            configs[cfg] = {"checked": False, "error": r.get("error", "not run")}
-            continue
-        configs[cfg] = {"value": round(r["value"], 2), "unit": r["unit"], "kernel_ms": round(r["kernel_ms"], 4), "bound": r["roofline"]["bound"],
-                        "frac": r["roofline"]["frac"], "checked": r["checked"], "kernel": r["kernel"],
-                        "cpu_baseline": (r.get("cpu_baseline") or {}).get("value"), "cpu_unit": (r.get("cpu_baseline") or {}).get("unit")}
-    others.sort(key=lambda r: 0 if r.get("workload", "").startswith("device ceilings") else 1)
-    line = {
-        "other_workloads": others,
-        "metric": "GEMM TFLOP/s + % MFMA peak; elementwise/transpose GB/s + % HBM peak (1 GPU)",
-        "value": round(main_res["value"], 2), "unit": main_res["unit"], "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
-        "ms_per_step": round(main_res["ms_per_step"], 4), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": main_res["dtype"], "data": "synthetic",
-        "config": {"workload": main_res["workload"], "kernel": main_res["kernel"], "kernel_ms": round(main_res["kernel_ms"], 4),
-                   "inputs": main_res["inputs"], "checked": main_res["checked"], "check": main_res["check"],
-                   "buffers": "4 rotating sets (1 GiB) so reads miss the Infinity Cache" if main_res["unit"] == "GB/s" else "single set",
-                   "configs": configs, **({"programs": main_res["programs"]} if "programs" in main_res else {})},
-        "roofline": main_res["roofline"],
-        "cpu_baseline": main_res.get("cpu_baseline"),
-    }
-    print(json.dumps(line))
+    for r in others:
+        print(json.dumps(r), file=sys.stderr, flush=True)
+    print(json.dumps(summary_line(args, main_res, dict([(args.workload, main_res)] + list(zip(other_names, others))))), flush=True)
 
 
 if __name__ == "__main__":

@@ -171,7 +171,7 @@ struct Signature {
   int in_dtype[kJitInputs], in_kind[kJitInputs];
   int out_dtype = 0;
   bool narrow = true;
-  bool ragged = false;       // the width is not a multiple of 8: the last vector of every row moves element by element
+  bool ragged = false;       // the width is not a multiple of 8: the last vector of every row is loaded whole and stored element by element
   bool tiled = false;        // an operand is column-major: 64 x 64 tiles, such operands staged through LDS
   bool rowwise = false;      // the program reduces along rows: the row skeleton, compiled for one (threads, chunks) shape
   int threads = 256, chunks = 1;

@@ -641,8 +641,8 @@ bool match_fused_row(const RowBuilder &B, const StackProgram &SP, const kapy_glo
 
 int run_row_program(const kapy_ew_inst *prog, int n_inst, const int *result_dtype, const kapy_global *const *ins, int n_ins, const kapy_global *out,
                     hipStream_t stream) {
-  const char *why = "elementwise: a program with a reduce needs axis 1, contiguous rows of a multiple of 8 and at most 32768 elements, zero "
-                    "padding, full / row / column / scalar operands of float type, one st_global and at most three row values in flight";
+  const char *why = "elementwise: a program with a reduce needs axis 1, contiguous rows of at most 32768 elements and a multiple of 8 (any number above 256 for "
+                    "a 16-bit softmax), zero padding, full / row / column / scalar operands of float type, one st_global and at most three row values in flight";
   RowBuilder B;
   int reg[kMaxRegs];
   for (int r = 0; r < kMaxRegs; ++r) reg[r] = -1;

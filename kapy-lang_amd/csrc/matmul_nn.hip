@@ -1,4 +1,5 @@
-// matmul_nn.hip — the tiled kernel for 16-bit operands of which at least one is contiguous along its other extent (128 x 128 tiles).
+// matmul_nn.hip — the tiled kernel for 16-bit operands of which at least one is contiguous along its other extent, or whose lines end
+// inside a 16-byte piece (128 x 128 tiles).
 #include "matmul_tile.hpp"
 #include "operand_pieces.hpp"
 
@@ -6,21 +7,16 @@ namespace kapy {
 namespace {
 
 // ---------------------------------------------------------------------------------------------
-// NN kernel: lhs row-major (K contiguous), rhs row-major (N contiguous), extents multiples of the
-// 128 x 128 x BK tile.  4 wavefronts (2x2), wave tile 64x64 = 4x4 blocks of the 16x16x32 instruction.
-// The rhs tile is staged as it lies in memory, [BK][128] with N contiguous, by the same LDS-direct
-// buffer loads as the lhs; the K-contiguous operand registers the matrix instruction wants are made
-// on the way out of LDS by ds_read_b64_tr_b16: a 16-lane group hands in 16 addresses of 8 bytes
-// (4 k-rows x 16 columns) and lane i gets column i of the four rows.  This replaces the
-// ldmatrix.trans of the reference (LdMatrixOpToLLVM.cpp:128-129).
+// NN kernel: 128 x 128 x BK tiles of operands in any layout with 16-byte aligned lines along the contiguous axis (A_TR / B_TR below),
+// any N and K, any M of a K-contiguous lhs, M a multiple of 8 of a transposed one.  4 wavefronts (2x2), wave tile 64x64 = 4x4
+// blocks of the 16x16x32 instruction.  An operand tile is staged as it lies in memory - a transposed one as [BK][128] - by
+// LDS-direct buffer loads; the K-contiguous operand registers that the matrix instruction wants of a transposed operand are
+// made on the way out of LDS by ds_read_b64_tr_b16: a 16-lane group hands in 16 addresses of 8 bytes (4 k-rows x 16 columns) and
+// lane i gets column i of the four rows.  This replaces the ldmatrix.trans of the reference (LdMatrixOpToLLVM.cpp:128-129).
 // STAGES-deep ring; the barrier at the top of iteration kt publishes tile kt+1 and frees the stage of
 // tile kt-1 for the loads of tile kt+STAGES-1.  Loads past the end of K re-read the last tile into
 // a stage nobody reads again, so every iteration is identical.
 constexpr int kNBM = 128, kNBN = 128;
-// rhs image: 16-byte chunk c of k-row r sits at chunk c ^ rhs_key(r).  A transposing read of a half
-// wave touches rows {0..3} + 8*{0,1} (+4) of a 32-row slice, 32 bytes of each: the key sends those
-// eight to the eight 32-byte bank groups of the 256-byte row.
-__device__ __forceinline__ uint32_t rhs_key(uint32_t row) { return ((row & 3) + 4 * ((row >> 3) & 1)) * 2; }
 
 // A_TR / B_TR: how each operand lies in memory and in LDS.  false: K-contiguous (a row-major lhs, a column-major rhs): rows
 // of BK elements staged under the tiled kernel's swizzle and read 16 bytes per lane.  true: contiguous along its other
@@ -65,7 +61,7 @@ __global__ __launch_bounds__(256) void nn_kernel(GemmParams p) {
     uint32_t chunk;
     if (tr) {
       line = o / kRowTr;
-      chunk = ((o % kRowTr) / 16) ^ rhs_key(line);
+      chunk = ((o % kRowTr) / 16) ^ transposed_key(line);
     } else {
       LA::locate(o, line, chunk);
     }
@@ -144,7 +140,7 @@ __global__ __launch_bounds__(256) void nn_kernel(GemmParams p) {
   const OperandLane frag_at = operand_lane(T::kShape, lane);
   const uint32_t grp = frag_at.k0 / T::kShape.kpack, l16 = frag_at.row;
   static_assert((16 * kRowKc) % (256 * LA::kLineParam) == 0, "an operand block must span whole swizzle periods");
-  const uint32_t tr_row = 8 * grp + (l16 >> 2), tr_key = rhs_key(tr_row);  // the key is the same for every kk and h
+  const uint32_t tr_row = 8 * grp + (l16 >> 2), tr_key = transposed_key(tr_row);  // the key is the same for every kk and h
   // Byte offset, inside an operand's image of a stage, of this lane's read for block `blk` (transposed) or slice kk (K-contiguous)
   // of the wave's half `w` of the operand.
   auto tr_off = [&](int w, int blk) { return tr_row * kRowTr + (((w * 8 + blk * 2 + ((l16 & 3) >> 1)) ^ tr_key) * 16) + (l16 & 1) * 8; };

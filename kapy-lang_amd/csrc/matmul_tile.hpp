@@ -55,14 +55,8 @@ struct TileLayout {
 // kernel's own waits and barriers.  The result is pending until the wait below has been executed: every
 // register that holds a pending result is an in/out operand of that wait, so the compiler sees each later
 // use as a use of the WAIT's result and cannot place it (or a copy feeding it) before the wait.
+// From LDS byte address `addr` + IMM (below 64 KiB), the immediate in the instruction: no address arithmetic.
 typedef uint32_t u32x2_lds __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ u32x2_lds tr_read_b64(const char *lds_ptr) {
-  const uint32_t addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)lds_ptr;  // LDS pointers are 32-bit byte offsets
-  u32x2_lds r;
-  asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r) : "v"(addr));
-  return r;
-}
-// The same from LDS byte address `addr` + IMM (below 64 KiB), the immediate in the instruction: no address arithmetic.
 template <uint32_t IMM>
 __device__ __forceinline__ u32x2_lds tr_read_b64_at(uint32_t addr) {
   static_assert(IMM < 65536, "a DS instruction's offset field has 16 bits");
@@ -77,6 +71,11 @@ __device__ __forceinline__ void tr_reads_wait(u32x2_lds (&h0)[4], u32x2_lds (&h1
                :
                : "memory");
 }
+
+// An operand contiguous along its other extent is staged as k-rows of 128 elements, 16-byte chunk c of k-row r at chunk
+// c ^ transposed_key(r).  A transposing read of a half wave touches rows {0..3} + 8*{0,1} (+4) of a 32-row slice, 32 bytes of each: the
+// key sends those eight to the eight 32-byte bank groups of the 256-byte row.
+__device__ __forceinline__ uint32_t transposed_key(uint32_t row) { return ((row & 3) + 4 * ((row >> 3) & 1)) * 2; }
 
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>): a loop whose counter is a compile-time constant in the body
 template <typename F, int... I>

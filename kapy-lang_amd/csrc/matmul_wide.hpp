@@ -5,7 +5,7 @@
 // 4 wavefronts (2 x 2) with a wave tile of 128 x BN/2.  An operand is staged as it lies in memory by LDS-direct buffer loads (the
 // cp_async of CpAsyncOpToLLVM.cpp:22-186).  K-contiguous (a row-major lhs, a column-major rhs): rows of 128 bytes under the tiled
 // kernel's swizzle, read 16 bytes per lane.  Contiguous along its other extent (a column-major lhs, a row-major rhs): for each 128
-// rows or columns an image [64 k-rows][128 elements] with 16-byte chunk c of k-row r at chunk c ^ wide_key(r), the operand registers
+// rows or columns an image [64 k-rows][128 elements] with 16-byte chunk c of k-row r at chunk c ^ transposed_key(r), the operand registers
 // made on the way out of LDS by ds_read_b64_tr_b16 (the ldmatrix.trans of LdMatrixOpToLLVM.cpp:128-129).
 //
 // One barrier per K-tile, before the tile's second and last K-slice: by then every wave holds that slice's fragments, so the stage is
@@ -24,10 +24,6 @@
 
 namespace kapy {
 namespace {
-
-// (a transposing read of a half wave touches k-rows {0..3} + 8*{0,1} (+4) of a 32-row slice, 32 bytes of each: the key sends
-// those eight to the eight 32-byte bank groups of the 256-byte row)
-__device__ __forceinline__ uint32_t wide_key(uint32_t row) { return ((row & 3) + 4 * ((row >> 3) & 1)) * 2; }
 
 // Waits for the transposing reads whose results sit in h0[j], h1[j] and hands those registers back as its own results (the
 // registers of a read still pending must not be touched by anything before this).
@@ -96,7 +92,7 @@ __global__ __launch_bounds__(256) void wide_kernel(GemmParams p) {
   const uint32_t my_byte = (uint32_t)wave * 1024u + lane * 16u;
   uint32_t kc_row, kc_chunk;
   L::locate(my_byte, kc_row, kc_chunk);
-  const uint32_t tr_krow = my_byte / kRowTr, tr_chunk = ((my_byte % kRowTr) / 16) ^ wide_key(tr_krow);
+  const uint32_t tr_krow = my_byte / kRowTr, tr_chunk = ((my_byte % kRowTr) / 16) ^ transposed_key(tr_krow);
   // (the lines and pieces a tile that hangs over an edge reads in place of those that do not exist: operand_pieces.hpp)
   using PiecesA = OperandPieces<A_TR, BK, EB>;
   using PiecesB = OperandPieces<B_TR, BK, EB>;
@@ -144,7 +140,7 @@ __global__ __launch_bounds__(256) void wide_kernel(GemmParams p) {
   // (transposed: the key enters by XOR); the rest is an immediate.
   const OperandLane frag_at = operand_lane(T::kShape, lane);
   const uint32_t grp = frag_at.k0 / T::kShape.kpack, l16 = frag_at.row;
-  const uint32_t tr_row = 8 * grp + (l16 >> 2), tr_key = wide_key(tr_row);  // (the key is the same for every slice and half)
+  const uint32_t tr_row = 8 * grp + (l16 >> 2), tr_key = transposed_key(tr_row);  // (the key is the same for every slice and half)
   auto tr_at = [&](int first, int blk) -> uint32_t {  // `first`: the wave's first row or column of the tile
     return (first / 128) * kHalfTr + tr_row * kRowTr + ((((first % 128) / 8 + blk * 2 + ((l16 & 3) >> 1)) ^ tr_key) * 16) + (l16 & 1) * 8;
   };

@@ -52,7 +52,7 @@ def test_no_kernel_spills(tmp_path):
     assert objects, "no gfx950 code object found in the library"
     if os.path.exists(PROBE_LIB):
         objects += _code_objects(tmp_path, PROBE_LIB, "q")
-    seen, bad = 0, []
+    seen, families, bad = 0, set(), []
     for path in objects:
         notes = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes", path], check=True, capture_output=True, text=True).stdout
         for kernel in notes.split("- .agpr_count:")[1:]:
@@ -64,11 +64,12 @@ def test_no_kernel_spills(tmp_path):
             m = re.search(r"tn_kernel<.*, (true|false), (true|false), (true|false)>", name)
             if m and (m.group(1) == "false" or m.group(2) == "true"):  # element-store epilogue / partial last K-tile
                 continue
-            if "nn_kernel<" in name or "nn256_kernel<" in name:
+            families |= {f for f in ("tn_kernel<", "nn_kernel<", "wide_kernel<") if f in name}
+            if "nn_kernel<" in name or "wide_kernel<" in name:
                 # no register of any build may be spilled: a transposing read's result is pending until the kernel's own wait, and a
                 # spill (or a fragment buffer kept in scratch memory) would store it before it has arrived.  The builds with the
                 # element-store epilogue call that store out of line, which takes a private segment and nothing else.
-                packed = re.search(r"nn_kernel<[^,]+, \d+, \d+, true,", name) is not None or "nn256_kernel<" in name
+                packed = re.search(r"nn_kernel<[^,]+, \d+, \d+, true,", name) is not None or "wide_kernel<" in name
                 if int(field("vgpr_spill_count")) or int(field("sgpr_spill_count")) > 64 or int(field("private_segment_fixed_size")) > (0 if packed else 256):
                     bad.append("%s: %s VGPRs spilled, %s SGPRs spilled, %s bytes of private segment" %
                                (name[:140], field("vgpr_spill_count"), field("sgpr_spill_count"), field("private_segment_fixed_size")))
@@ -79,6 +80,7 @@ def test_no_kernel_spills(tmp_path):
                 bad.append("%s: %s VGPRs spilled, %s SGPRs spilled, %s bytes of private segment" %
                            (name[:140], field("vgpr_spill_count"), field("sgpr_spill_count"), field("private_segment_fixed_size")))
     assert seen > 100, "only %d kernels found" % seen
+    assert len(families) == 3, "of the matmul kernels only %s were found" % sorted(families)
     assert not bad, "\n".join(bad)
 
 

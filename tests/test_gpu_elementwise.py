@@ -226,7 +226,7 @@ def test_register_stack_kernel_tree_shapes_and_operand_kinds(ko):
 @pytest.mark.parametrize("which", ["gelu row bias", "gelu full bias", "x + y", "x*y + x"])
 def test_rows_with_a_ragged_last_vector_keep_the_fast_kernels_and_stay_inside_the_view(ko, width, which):
     """Views whose rows start 16-byte aligned but whose width is not a multiple of 8 (a sub-view of a wider tensor): the
-    last vector of every row moves element by element; nothing outside the view is read into the result or written."""
+    last vector of every row is loaded whole and stored element by element; nothing outside the view reaches the result or is written."""
     m, pitch = 37, 2048
     xp = ko.fill_normal(m * pitch, kh.F16, 101).reshape(m, pitch)
     yp = ko.fill_normal(m * pitch, kh.F16, 102).reshape(m, pitch)

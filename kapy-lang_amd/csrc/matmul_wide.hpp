@@ -13,9 +13,10 @@
 // instructions of that last slice, with the next tile's first slice to land.  Three stages of 48 KiB (256 x 128): half of them
 // there, half in the first slice of the next tile, with a whole tile time more to land - its slices are half as long.
 //
-// What bounds it: 256 x 256, the matrix cores at the clock the power limit leaves (LDS reads and writes take 0.75 of the matrix
-// time); 256 x 128, LDS traffic at 1.1 of the matrix time (128 x 128 tiles: 1.5) and, on operands that come from HBM, the loads the
-// LDS has room to keep in flight.  Measured, 128 x 128 tiles (or the operands turned first) -> here: fp8 1000 x 8192 x 8192 60 -> 53 us;
+// What bounds it: 256 x 256, the matrix cores at the clock the power limit leaves (matrix pipe busy for 88 % of the wave clocks at
+// 8192^3); 256 x 128 with one tile per CU, what nothing else on that CU covers - first loads, epilogue, waits for loads (matrix pipe busy
+// for 73 .. 75 % of the wave clocks with 64 K-tiles; LDS reads for 0.41 of the matrix clocks, 0.26 on 256 x 256 tiles; no bank
+// conflicts in the loop).  Measured, 128 x 128 tiles (or the operands turned first) -> here: fp8 1000 x 8192 x 8192 60 -> 52 us;
 // bf16 2048 x 4096 x 4096 row-major 63.5 -> 54, two transposed operands 66 -> 56; 8192^3 with two transposed operands, fp32 result,
 // 0.84 ms for the turns and the product -> 0.74.
 #pragma once

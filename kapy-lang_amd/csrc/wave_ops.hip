@@ -245,8 +245,8 @@ __global__ __launch_bounds__(256) void reduce_rows_short_kernel(ReduceParams p) 
 }
 
 // The last-arrived workgroup's fold of `chunks` partial lines for COLS kept indices starting at keep0: the 256 lanes form
-// 256 / COLS groups that take chunks g, g + groups, ... (sixteen loads in flight per lane), the groups meet in LDS and are
-// folded in group order.  part: [256 / COLS][COLS + 1] floats.
+// 256 / COLS groups that take chunks g, g + groups, ... (sixteen loads in flight per lane while a group has sixteen chunks left, one
+// at a time after that), the groups meet in LDS and are folded in group order.  part: [256 / COLS][COLS + 1] floats.
 template <int COLS, int KIND>
 __device__ __forceinline__ void fold_partial_lines(const ReduceParams &p, const Shared &sh, int64_t keep0, int32_t chunks, float *part) {
   constexpr int GROUPS = 256 / COLS;

@@ -55,37 +55,30 @@ __global__ __launch_bounds__(256) void nn_kernel(GemmParams p) {
   // and pieces that do not exist (operand_pieces.hpp).
   using PiecesA = OperandPieces<A_TR, BK, 2>;
   using PiecesB = OperandPieces<B_TR, BK, 2>;
-  // row or k-row, and first element along it, of the piece that instruction q of an operand brings this lane
-  auto piece_of = [&](bool tr, int q, uint32_t &line, uint32_t &first) {
-    const uint32_t o = (uint32_t)(wave + q * 4) * 1024u + lane * 16u;
-    uint32_t chunk;
-    if (tr) {
-      line = o / kRowTr;
-      chunk = ((o % kRowTr) / 16) ^ transposed_key(line);
-    } else {
-      LA::locate(o, line, chunk);
-    }
-    first = chunk * 8;
-  };
+  // Row (k-row) and first element along it of the piece that instruction 0 brings this lane; instruction q's is as many rows further on
+  // as 4 KiB hold (no key mixes in a bit that q changes).
+  constexpr int kStepKc = 4096 / kRowKc, kStepTr = 4096 / kRowTr;
+  static_assert(16 % LA::kLineParam == 0 && kStepTr % 16 == 0, "the pieces of one lane must lie at one place along their rows");
+  const uint32_t my_byte = (uint32_t)wave * 1024u + lane * 16u;
+  uint32_t kc_row, kc_chunk;
+  LA::locate(my_byte, kc_row, kc_chunk);
+  const uint32_t tr_krow = my_byte / kRowTr, tr_chunk = ((my_byte % kRowTr) / 16) ^ transposed_key(tr_krow);
+  const uint32_t a_first = (A_TR ? tr_chunk : kc_chunk) * 8, b_first = (B_TR ? tr_chunk : kc_chunk) * 8;
+  const uint32_t a_line0 = (A_TR ? tr_krow : kc_row) * (uint32_t)a_ld, b_line0 = (B_TR ? tr_krow : kc_row) * (uint32_t)b_ld;
   uint32_t a_goff[kLoadsOp], b_goff[kLoadsOp];
 #pragma unroll
   for (int q = 0; q < kLoadsOp; ++q) {
-    uint32_t line, first;
-    piece_of(A_TR, q, line, first);
-    a_goff[q] = PiecesA::lane(line, first, a_ld, p.M - m0);
-    piece_of(B_TR, q, line, first);
-    b_goff[q] = PiecesB::lane(line, first, b_ld, p.N - n0);
+    a_goff[q] = PiecesA::lane(a_line0 + (uint32_t)(q * (A_TR ? kStepTr : kStepKc) * a_ld), a_first, a_ld, p.M - m0);
+    b_goff[q] = PiecesB::lane(b_line0 + (uint32_t)(q * (B_TR ? kStepTr : kStepKc) * b_ld), b_first, b_ld, p.N - n0);
   }
   // From the last K-tile on (the loads past the end of K repeat it): pieces at or beyond K get an offset no descriptor covers.
+  // (a K-contiguous operand's line does not matter here: its first element is its K position)
   auto enter_k_tail = [&]() __attribute__((always_inline)) {
     const int32_t k_left = p.K - (KT - 1) * BK;
 #pragma unroll
     for (int q = 0; q < kLoadsOp; ++q) {
-      uint32_t line, first;
-      piece_of(A_TR, q, line, first);
-      a_goff[q] = PiecesA::beyond_k(line, first, k_left) ? PiecesA::kNowhere : a_goff[q];
-      piece_of(B_TR, q, line, first);
-      b_goff[q] = PiecesB::beyond_k(line, first, k_left) ? PiecesB::kNowhere : b_goff[q];
+      a_goff[q] = PiecesA::beyond_k(tr_krow + q * kStepTr, a_first, k_left) ? PiecesA::kNowhere : a_goff[q];
+      b_goff[q] = PiecesB::beyond_k(tr_krow + q * kStepTr, b_first, k_left) ? PiecesB::kNowhere : b_goff[q];
     }
   };
   // (KTAIL) Of a K-contiguous operand the piece that K ends inside has arrived with what lies behind K: this lane's copy of it in the
@@ -96,11 +89,9 @@ __global__ __launch_bounds__(256) void nn_kernel(GemmParams p) {
 #pragma unroll
     for (int q = 0; q < kLoadsOp; ++q) {
       char *piece = lds + stage * kStage + q * 4096 + wave * 1024 + lane * 16;
-      uint32_t line, first;
-      piece_of(false, q, line, first);
 #pragma unroll
       for (int e = 1; e < 8; ++e) {
-        const int32_t from = k_left - (int32_t)first;   // (one compare per element: the piece K ends inside has 1 .. 7 left)
+        const int32_t from = k_left - (int32_t)kc_chunk * 8;   // (one compare per element: the piece K ends inside has 1 .. 7 left)
         if (from > 0 && from <= e) {
           if constexpr (!A_TR) ((uint16_t *)piece)[e] = 0;
           if constexpr (!B_TR) ((uint16_t *)(piece + kBytesA))[e] = 0;

@@ -58,13 +58,13 @@ __global__ __launch_bounds__(64 * WM * WN) void tn_kernel(GemmParams p) {
   for (int i = 0; i < C::kLoadsAPerWave; ++i) {
     uint32_t row, chunk;
     L::locate((uint32_t)(wave + i * C::kWaves) * 1024u + lane * 16u, row, chunk);
-    a_goff[i] = Pieces::lane(row, chunk * Pieces::kPer, (int32_t)p.a_sm, kRowsReplaced ? p.M - m0 : BM);
+    a_goff[i] = Pieces::lane(row * (uint32_t)p.a_sm, chunk * Pieces::kPer, (int32_t)p.a_sm, kRowsReplaced ? p.M - m0 : BM);
   }
 #pragma unroll
   for (int i = 0; i < C::kLoadsBPerWave; ++i) {
     uint32_t row, chunk;
     L::locate((uint32_t)(wave + i * C::kWaves) * 1024u + lane * 16u, row, chunk);
-    b_goff[i] = Pieces::lane(row, chunk * Pieces::kPer, (int32_t)p.b_sn, kRowsReplaced ? p.N - n0 : BN);
+    b_goff[i] = Pieces::lane(row * (uint32_t)p.b_sn, chunk * Pieces::kPer, (int32_t)p.b_sn, kRowsReplaced ? p.N - n0 : BN);
   }
   const char *a_tile = p.a + (int64_t)m0 * p.a_sm * EB;
   const char *b_tile = p.b + (int64_t)n0 * p.b_sn * EB;

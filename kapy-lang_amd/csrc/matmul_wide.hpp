@@ -100,10 +100,11 @@ __global__ __launch_bounds__(256) void wide_kernel(GemmParams p) {
   auto line_of = [&](bool tr, int q) -> uint32_t { return tr ? tr_krow + 16 * (q % 4) : kc_row + 32 * q; };
   auto first_of = [&](bool tr, int q) -> uint32_t { return tr ? tr_chunk * 8 + 128 * (q / 4) : kc_chunk * (16 / EB); };
   uint32_t a_goff[kLoadsA], b_goff[kLoadsB];
+  const uint32_t a_line0 = line_of(A_TR, 0) * (uint32_t)a_ld, b_line0 = line_of(B_TR, 0) * (uint32_t)b_ld;
 #pragma unroll
-  for (int q = 0; q < kLoadsA; ++q) a_goff[q] = PiecesA::lane(line_of(A_TR, q), first_of(A_TR, q), a_ld, p.M - m0);
+  for (int q = 0; q < kLoadsA; ++q) a_goff[q] = PiecesA::lane(a_line0 + (uint32_t)((A_TR ? 16 * (q % 4) : 32 * q) * a_ld), first_of(A_TR, q), a_ld, p.M - m0);
 #pragma unroll
-  for (int q = 0; q < kLoadsB; ++q) b_goff[q] = PiecesB::lane(line_of(B_TR, q), first_of(B_TR, q), b_ld, p.N - n0);
+  for (int q = 0; q < kLoadsB; ++q) b_goff[q] = PiecesB::lane(b_line0 + (uint32_t)((B_TR ? 16 * (q % 4) : 32 * q) * b_ld), first_of(B_TR, q), b_ld, p.N - n0);
   auto enter_k_tail = [&]() __attribute__((always_inline)) {
     const int32_t k_left = p.K - (KT - 1) * BK;
 #pragma unroll

@@ -20,11 +20,12 @@ template <bool TR, int BK, int EB>
 struct OperandPieces {
   static constexpr int kPer = 16 / EB;  // elements per piece
   static constexpr uint32_t kNowhere = 0x7fffffffu;
-  static constexpr uint32_t lane(uint32_t line, uint32_t first, int32_t ld, int32_t left) {
-    const uint32_t last = (uint32_t)(left - 1);
+  // (`line_at`: line * ld, so that a loader forms it once and steps it from load to load)
+  static constexpr uint32_t lane(uint32_t line_at, uint32_t first, int32_t ld, int32_t left) {
+    const uint32_t last = (uint32_t)(left - 1), last_at = last * (uint32_t)ld;
     if (TR) first = first < last ? first : last / kPer * kPer;
-    else line = line < last ? line : last;
-    return (line * (uint32_t)ld + first) * EB;
+    else line_at = line_at < last_at ? line_at : last_at;
+    return (line_at + first) * EB;
   }
   // whether the whole piece lies at or beyond K, of which k_left positions are in the last K-tile
   static constexpr bool beyond_k(uint32_t line, uint32_t first, int32_t k_left) { return (int32_t)(TR ? line : first) >= k_left; }

@@ -30,7 +30,7 @@ static void walk(int width, int left, int k, int64_t ld) {
           if (scalar > bytes) die("the scalar part lies beyond the operand", j, line, first, scalar);
           continue;
         }
-        const int64_t lane = P::lane((uint32_t)line, (uint32_t)first, (int32_t)ld, left), at = scalar + lane;
+        const int64_t lane = P::lane((uint32_t)line * (uint32_t)ld, (uint32_t)first, (int32_t)ld, left), at = scalar + lane;
         if (at < 0 || at + 16 > bytes) die("read outside the operand", j, line, first, at);
         if (lane >= bytes || lane >= bytes - scalar) die("an existing piece fails the range check", j, line, first, at);
         const int jj = last ? tiles - 1 : j;
@@ -51,7 +51,7 @@ static void walk_rows(int width, int rows, int k, int64_t ld) {
   for (int j = 0; j < tiles; ++j)
     for (int line = left; line < width; ++line)
       for (int first = 0; first < BK; first += 16 / EB, ++checked) {
-        const int64_t lane = P::lane((uint32_t)line, (uint32_t)first, (int32_t)ld, width), scalar = P::tile(j, tiles, (int32_t)ld);
+        const int64_t lane = P::lane((uint32_t)line * (uint32_t)ld, (uint32_t)first, (int32_t)ld, width), scalar = P::tile(j, tiles, (int32_t)ld);
         if (lane >= bytes - scalar && lane >= bytes && scalar <= bytes) continue;
         std::printf("a row that does not exist is in range: %d rows in tiles of %d, K %d, pitch %lld: K-tile %d row %d position %d\n", rows, width, k, (long long)ld, j, line, first);
         std::exit(1);

@@ -1068,8 +1068,8 @@ def pmc_summary(fetch_csv, write_csv):
 
     out = ["rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, all bench workloads, one MI355X (gfx950)", "",
            "commands (two runs, one counter each; from the repository root after `cd /tmp && export TMPDIR=/tmp && cd <repo>`):",
-           "  rocprofv3 --pmc FETCH_SIZE -d gpurun_out/prof/pmc_fetch -o pmc_fetch --output-format csv -- python3 bench.py --no-cpu --skip ceilings,mlir_fixtures --steps 3 --warmup 1",
-           "  rocprofv3 --pmc WRITE_SIZE -d gpurun_out/prof/pmc_write -o pmc_write --output-format csv -- python3 bench.py --no-cpu --skip ceilings,mlir_fixtures --steps 3 --warmup 1",
+           "  rocprofv3 --pmc FETCH_SIZE -d out/prof/pmc_fetch -o pmc_fetch --output-format csv -- python3 bench.py --no-cpu --skip ceilings,mlir_fixtures --steps 3 --warmup 1",
+           "  rocprofv3 --pmc WRITE_SIZE -d out/prof/pmc_write -o pmc_write --output-format csv -- python3 bench.py --no-cpu --skip ceilings,mlir_fixtures --steps 3 --warmup 1",
            "  python3 bench.py --pmc-summary <pmc_fetch counter_collection.csv> <pmc_write counter_collection.csv> > profiles/bench_all_workloads.hbm_traffic_pmc.txt",
            "", "Per-dispatch mean of the counter (rocprofv3 reports KiB), by kernel and grid size (work-items); n = dispatches seen.", "",
            "%-86s %10s %20s %20s" % ("kernel", "grid", "FETCH_SIZE (n)", "WRITE_SIZE (n)")]
@@ -1122,7 +1122,7 @@ def stats_summary(stats_csv):
         return n.replace("void ", "").replace("kapy::(anonymous namespace)::", "").replace("kapy::", "").split("(")[0]
     out = ["rocprofv3 kernel statistics, all bench workloads, one MI355X (gfx950)", "",
            "commands (from the repository root, after `cd /tmp && export TMPDIR=/tmp && cd <repo>`):",
-           "  rocprofv3 --kernel-trace --stats -d gpurun_out/prof/stats_all -o stats_all --output-format csv -- python3 bench.py --no-cpu --skip ceilings",
+           "  rocprofv3 --kernel-trace --stats -d out/prof/stats_all -o stats_all --output-format csv -- python3 bench.py --no-cpu --skip ceilings",
            "  python3 bench.py --stats-summary <stats_all_kernel_stats.csv> > profiles/bench_all_workloads.kernel_stats.txt", "",
            "Rows of this library's kernels (torch's fill / compare kernels omitted).  Calls include the untimed clock pre-warm launches of",
            "bench.py.  kapy_ew_flat_* / kapy_ew_rows_* are the kernels kapy_elementwise compiled at run time in that process (the name ends in",
@@ -1138,8 +1138,8 @@ def ceilings_summary(bench_json):
     res = json.loads(open(bench_json).read().strip().split("\n")[-1])
     out = ["Device ceilings measured by the probe library's kernels (libkapy_probe.so) and the tiled GEMMs' fixed cost per launch, one MI355X (gfx950)", "",
            "commands (from the repository root):",
-           "  python3 bench.py --no-cpu --no-others --workload ceilings > gpurun_out/ceilings.json",
-           "  python3 bench.py --ceilings-summary gpurun_out/ceilings.json > profiles/device_ceilings.probe_kernels.txt", "",
+           "  python3 bench.py --no-cpu --no-others --workload ceilings > out/ceilings.json",
+           "  python3 bench.py --ceilings-summary out/ceilings.json > profiles/device_ceilings.probe_kernels.txt", "",
            "bench.py's figures in that run (HIP events around back-to-back launches; the shader clock is what the kernel itself reads: s_memtime",
            "ticks of one wave against the 100 MHz s_memrealtime over the same interval)."]
 

@@ -478,10 +478,10 @@ int matmul_f8(const kapy_global *a, const kapy_global *b, const float *row_scale
   if (p.M == 0 || p.N == 0) return KAPY_OK;
   // K-contiguous operands with 16-byte aligned rows of whole 16-byte pieces: what the tiled kernel needs (its ring builds take
   // a partial last K-tile); the streaming kernels below need whole 128-byte K steps
-  // (and unsigned 32-bit row offsets: rows in reverse order go to the general kernels)
-  const bool k_pieces = p.a_sk == 1 && p.b_sk == 1 && vector_bytes(a, 1) == 16 && vector_bytes(b, 0) == 16 && p.K % 16 == 0 && p.K > 0 &&
-                        (p.M == 1 || p.a_sm >= 0) && (p.N == 1 || p.b_sn >= 0);
-  const bool k_contig = k_pieces && p.K % 128 == 0;
+  const bool k_pieces = p.a_sk == 1 && p.b_sk == 1 && vector_bytes(a, 1) == 16 && vector_bytes(b, 0) == 16 && p.K % 16 == 0 && p.K > 0;
+  // (all of them form unsigned 32-bit row offsets: rows in reverse order go to the general kernels)
+  const bool rows_forward = (p.M == 1 || p.a_sm >= 0) && (p.N == 1 || p.b_sn >= 0);
+  const bool k_contig = k_pieces && rows_forward && p.K % 128 == 0;
   // Many rows: the tiled LDS-direct kernel (MFMA-bound).  Few rows: the skinny kernel (HBM-bound).
   // With a workspace the tiled kernel can split K over several workgroups per tile, which fills the device at few rows too.
   kapy_matmul_cfg c = {KAPY_MATMUL_AUTO, 0, 0, 0, KAPY_RN, 0, 0, 0, nullptr, 0};
@@ -503,7 +503,7 @@ int matmul_f8(const kapy_global *a, const kapy_global *b, const float *row_scale
     if (rc) return rc;
     // an explicit split is a request for the tiled kernel; the library's own choice weighs it against the block kernel
     const int tiled_from = block_ok && c.split_k <= 1 ? (g.split_k > 1 ? kTiledFromMSplit : kTiledFromM) : (g.split_k > 1 ? kTiledFromMSplitNoBlock : kTiledFromMNoBlock);
-    if (k_contig && p.M < tiled_from) rc = KAPY_ERR_UNSUPPORTED;  // few rows: the streaming kernels below (which need whole K steps)
+    if (!rows_forward || (k_contig && p.M < tiled_from)) rc = KAPY_ERR_UNSUPPORTED;  // few rows: the streaming kernels below (which need whole K steps)
     else rc = matmul_f8_tiled(g, fmt_of(a->dtype), fmt_of(b->dtype), c.tile_m, c.tile_n, s);
     if (rc != KAPY_ERR_UNSUPPORTED) return rc;
   }

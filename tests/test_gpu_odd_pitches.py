@@ -68,6 +68,9 @@ def test_f8_single_row_of_any_pitch(ko, N, K):
 def test_operand_rows_in_reverse_order(ko, dt, M, N, K):
     for a_pitch, b_pitch in ((-K, K), (K, -K - 16), (-K, -K)):
         _check(ko, dt, M, N, K, a_pitch, b_pitch, kh.F32, 1e-4 if kh.DTYPE_BYTES[dt] == 1 else 1e-5, 87)
+    if kh.DTYPE_BYTES[dt] == 1:   # a split that is none is refused here as well
+        with pytest.raises(kh.KapyError):
+            _check(ko, dt, M, N, K, -K, K, kh.F32, 1e-4, 88, split_k=-1)
 
 
 @pytest.mark.parametrize("out", [kh.F32, kh.F16])

@@ -19,10 +19,11 @@ namespace kapy {
 template <bool TR, int BK, int EB>
 struct OperandPieces {
   static constexpr int kPer = 16 / EB;  // elements per piece
+  static constexpr int32_t kLines = 256;  // no tile has more rows or columns: the offset of the last existing one inside it fits 32 bits
   static constexpr uint32_t kNowhere = 0x7fffffffu;
   // (`line_at`: line * ld, so that a loader forms it once and steps it from load to load)
   static constexpr uint32_t lane(uint32_t line_at, uint32_t first, int32_t ld, int32_t left) {
-    const uint32_t last = (uint32_t)(left - 1), last_at = last * (uint32_t)ld;
+    const uint32_t last = (uint32_t)(left < kLines ? left : kLines) - 1u, last_at = last * (uint32_t)ld;
     if (TR) first = first < last ? first : last / kPer * kPer;
     else line_at = line_at < last_at ? line_at : last_at;
     return (line_at + first) * EB;

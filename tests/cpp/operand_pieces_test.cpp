@@ -78,6 +78,12 @@ static void walk_all(int width) {
 }
 
 int main() {
+  // operands of 2^32 elements and more behind the tile
+  for (int rows : {(1 << 19) + 1, (1 << 19) + 40, 1 << 20}) {
+    walk<false, 64, 2>(256, rows, 192, 8192);
+    walk<true, 64, 2>(256, rows, 192, (1 << 20));
+    walk<false, 128, 1>(256, rows, 384, 8192);
+  }
   for (int width : {64, 128, 256}) {
     walk_all<64, 2>(width);
     walk_all<32, 2>(width);
